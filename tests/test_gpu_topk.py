@@ -311,3 +311,35 @@ def test_pool_bound_and_full_ranking():
                                             "bfloat16")
             assert got == flat, f"beam {beam} request {q}"
             b += r
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,v,beam", [(1, 7, 1), (1, 5, 2), (2, 1021, 4), (3, 257, 8), (2, 2047, 16), (4, 4100, 4), (1, 6145, 32),
+                                      (2, 10007, 2), (4, 32000, 4), (8, 128256, 8), (2, 70001, 64)])
+def test_few_rows_and_short_segments(dtype, n, v, beam):
+    """Few rows (split into segments no shorter than a chunk per thread) and
+    vocabularies that leave waves of a segment partly or wholly without
+    logits: the candidate thresholds come from the waves that hold some."""
+    say(f"topk few rows {n} x {v} beam {beam} {dtype}")
+    g = torch.Generator().manual_seed(n * 7 + v)
+    logits = (torch.randn((n, v), generator=g) * 2.0).to(dtype)
+    compare(logits, [-0.25 * i for i in range(n)], beam)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_segment_with_more_candidates_than_its_space(dtype):
+    """One wave of a segment holds far smaller logits than the others (the
+    shares of k let too many positions through, the tighter threshold does
+    not), and a row whose large values crowd into a few threads (the
+    tighter threshold overflows too: the exact selection)."""
+    say(f"topk crowded segments {dtype}")
+    g = torch.Generator().manual_seed(31)
+    v = 64000
+    x = torch.randn((4, v), generator=g) * 2.0
+    per = 4 if dtype == torch.float32 else 8
+    lane = (torch.arange(v) // per) % 256
+    x[0, lane < 64] -= 40.0
+    x[1, (lane >= 64) & (lane < 128)] -= 400.0
+    x[2, lane % 64 == 3] += 30.0
+    x[3, :3000] += 50.0
+    compare(x.to(dtype), [0.0, -0.5, -1.0, -1.5], 8)
