@@ -181,8 +181,16 @@ class _PagedPlanner:
             # (a capacity error with plan_ints 0 is a fixed layout's, which no
             # buffer size cures: MemoryError)
             _lib.check(rc, "attention plan")
+            if info.kernel == 2 and info.stream_loop == 2 and self._need(info) > self._ws.numel():
+                flags |= _lib.BE_PLAN_NO_BLOCKS       # the streaming plan's 16-bit slots may still fit
+                continue
             break
         self._install_plan(info, buf, staging, max_page, head_dim, sm_scale, q_data_type)
+
+    @staticmethod
+    def _need(info) -> int:
+        """Workspace bytes of a plan: its words, then the partial rows."""
+        return (int(info.plan_ints) * 4 + _WS_ALIGN - 1) // _WS_ALIGN * _WS_ALIGN + int(info.partial_bytes)
 
     def _plan_flags(self) -> int:
         return (_lib.BE_PLAN_FORCE_VALU if self._force_valu else 0) | \
@@ -205,7 +213,7 @@ class _PagedPlanner:
         ``plan_ints`` words itself, before the next run."""
         plan_bytes = int(info.plan_ints) * 4
         part_off = (plan_bytes + _WS_ALIGN - 1) // _WS_ALIGN * _WS_ALIGN
-        need = part_off + int(info.partial_bytes)
+        need = self._need(info)
         if need > self._ws.numel():
             raise MemoryError(f"attention plan needs {need} workspace bytes, buffer has {self._ws.numel()}")
         key = (plan_bytes, need)
@@ -364,9 +372,10 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedPlanner):
     reference's prefill, models/modeling_llama.py:213-283, 775-798): request
     r's queries ``q[qo_indptr[r]:qo_indptr[r+1]]`` attend to its pages, whose
     K/V the caller wrote first; ``causal=True`` gives query i of n the first
-    kv_len - n + i + 1 tokens.  Runs on the MFMA tile kernel (bf16 / fp16) or
-    the VALU kernel (fp32) with a per-row causal limit; query tiles stop at
-    the chunk holding their last visible token."""
+    kv_len - n + i + 1 tokens.  bf16 / fp16 prompts run as 128-row MFMA blocks
+    (short ones of head_dim 128 on the streaming kernel), fp32 on the VALU
+    kernel, with a per-row causal limit; query tiles stop at the chunk holding
+    their last visible token."""
 
     def __init__(self, float_workspace_buffer: torch.Tensor, kv_layout: str = "NHD"):
         super().__init__(float_workspace_buffer, kv_layout)

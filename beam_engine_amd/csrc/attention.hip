@@ -16,55 +16,9 @@
 #include <algorithm>
 #include <vector>
 
-#include "attention.h"
+#include "attn_tile.h"
 
 namespace be {
-
-// ------------------------------------------------------------------ plan layout
-// Device plan = int32 words:
-//   items      [num_items][8]   WorkItem
-//   q_index    [num_queries]     query ids referenced by items
-//   pages      [sum of level page lists]
-//   merge_q    [num_merge]       queries the merge kernel combines
-//   merge_ptr  [num_merge + 1]   CSR into merge_rows
-//   merge_rows [...]             partial rows of each merged query
-struct WorkItem {
-  int32_t q_begin;     // first entry of q_index
-  int32_t q_count;     // queries in the tile
-  int32_t page_begin;  // first entry of pages[] of the item's group
-  int32_t tok_begin;   // first group token covered (a multiple of 32)
-  int32_t tok_count;   // tokens covered, > 0
-  int32_t out_row;     // first partial row, or -1: write the final output
-  int32_t vis0;        // causal: group tokens its first query sees, unclamped (query j: vis0 + j); else kNoCausal
-  int32_t pad1;
-};
-constexpr int32_t kNoCausal = 0x3fffffff;
-static_assert(sizeof(WorkItem) == 32, "WorkItem is 8 int32 words");
-
-constexpr int kMaxRows = 32;       // rows (queries x GQA group) per VALU workgroup
-constexpr int kMaxTileRows = 128;  // rows per MFMA workgroup (8 row tiles of 16)
-
-struct AttnArgs {
-  const void* q;
-  int64_t q_sn, q_sh;
-  const void* kv;
-  void* out;
-  int64_t o_sn, o_sh;
-  float* out_lse;
-  float* part_o;      // [rows, Hq, D]
-  float* part_lse;    // [rows, Hq]
-  const WorkItem* items;
-  const int32_t* q_index;
-  const int32_t* pages;
-  // fused merge (null counters: the separate merge kernel runs instead)
-  const int32_t* q_merge;      // per query: merge-list index or -1
-  const int32_t* merge_ptr;    // CSR of partial rows per merge-list entry
-  const int32_t* merge_rows;
-  int32_t* counters;           // [num_merge][hkv] arrivals, zero between runs
-  const int32_t* live_items;   // fixed layout: live item count (surplus workgroups exit)
-  int page_size, hkv, hq, g;
-  float scale_log2;   // sm_scale * log2(e)
-};
 
 struct MergeArgs {
   const float* part_o;
@@ -78,80 +32,6 @@ struct MergeArgs {
   const int32_t* live;         // fixed layout: live entry count (surplus workgroups exit)
   int hq;
 };
-
-// Element offset of (page, kv, slot, head, 0) in a [P, 2, page, Hkv, D] layer.
-__device__ __forceinline__ int64_t kv_off(int page, int kvsel, int slot, int head, int page_size,
-                                          int hkv, int d) {
-  return ((((int64_t)page * 2 + kvsel) * page_size + slot) * hkv + head) * (int64_t)d;
-}
-
-// Writes the finished state of one row: o = acc / l, lse = (m + log2 l) ln 2.
-template <typename T>
-__device__ __forceinline__ void store_row_lse(const AttnArgs& a, const WorkItem& it, int j, int head,
-                                              float m2, float l) {
-  float lse = (l > 0.f) ? (m2 + log2f(l)) * 0.69314718055994531f : -INFINITY;
-  if (it.out_row < 0) {
-    if (a.out_lse) {
-      int qi = a.q_index[it.q_begin + j];
-      a.out_lse[(int64_t)qi * a.hq + head] = lse;
-    }
-  } else {
-    a.part_lse[(int64_t)(it.out_row + j) * a.hq + head] = lse;
-  }
-}
-
-// Fused split-K merge.  Called by every thread of a workgroup after it wrote
-// its partial rows.  For each query of the item the workgroup counts its
-// arrival on (query, kv head); the workgroup that completes the count merges
-// the g heads of that query from every partial row by log-sum-exp, writes the
-// output and resets the counter for the next run.  The release fence makes
-// this workgroup's partial rows visible device-wide (all XCD L2s) before its
-// arrival is counted; the acquire fence orders the merger's reads after it.
-template <typename T, int D>
-__device__ void fused_merge_epilogue(const AttnArgs& a, const WorkItem& it, int kvh, int* s_last) {
-  __threadfence();
-  __syncthreads();
-  const int tid = threadIdx.x;
-  if (tid < it.q_count) {
-    const int qi = a.q_index[it.q_begin + tid];
-    const int mi = a.q_merge[qi];
-    const int expect = a.merge_ptr[mi + 1] - a.merge_ptr[mi];
-    const int old = __hip_atomic_fetch_add(&a.counters[(int64_t)mi * a.hkv + kvh], 1, __ATOMIC_ACQ_REL,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    s_last[tid] = (old == expect - 1) ? mi : -1;
-  }
-  __syncthreads();
-  bool fenced = false;
-  for (int j = 0; j < it.q_count; ++j) {
-    const int mi = s_last[j];
-    if (mi < 0) continue;
-    if (!fenced) {
-      __threadfence();
-      fenced = true;
-    }
-    const int qi = a.q_index[it.q_begin + j];
-    const int rb = a.merge_ptr[mi], re = a.merge_ptr[mi + 1];
-    // thread -> (head hh, column d); g * D elements over 256 threads
-    for (int e = tid; e < a.g * D; e += 256) {
-      const int hh = e / D, d = e - hh * D, head = kvh * a.g + hh;
-      float M = -INFINITY;
-      for (int r = rb; r < re; ++r) M = fmaxf(M, a.part_lse[(int64_t)a.merge_rows[r] * a.hq + head]);
-      float z = 0.f, acc = 0.f;
-      if (M != -INFINITY) {
-        for (int r = rb; r < re; ++r) {
-          const int64_t row = (int64_t)a.merge_rows[r] * a.hq + head;
-          const float wgt = expf(a.part_lse[row] - M);
-          z += wgt;
-          acc += wgt * a.part_o[row * D + d];
-        }
-      }
-      T* op = reinterpret_cast<T*>(a.out) + (int64_t)qi * a.o_sn + (int64_t)head * a.o_sh;
-      op[d] = from_f32<T>(z > 0.f ? acc / z : 0.f);
-      if (d == 0 && a.out_lse) a.out_lse[(int64_t)qi * a.hq + head] = (z > 0.f) ? M + logf(z) : -INFINITY;
-    }
-    if (tid == 0) a.counters[(int64_t)mi * a.hkv + kvh] = 0;
-  }
-}
 
 // ================================================================== MFMA kernel
 // bf16/fp16 storage, D in {64, 128, 256}, up to 16*RT rows (queries x GQA
@@ -176,8 +56,6 @@ __device__ void fused_merge_epilogue(const AttnArgs& a, const WorkItem& it, int 
 // S^T tile gives lane (lg, lc) tokens 4*lg..4*lg+3 of row lc, which is exactly
 // the B operand (P^T) of v_mfma_f32_16x16x16 for O^T = V^T P^T, whose A
 // operand is 4 consecutive tokens of one head_dim row of the transposed V.
-constexpr int kTile = 64;              // tokens per LDS tile
-constexpr int kMaxPagesLds = 1024;     // page ids of one item staged in LDS
 
 template <int D>
 struct TileLds {
@@ -784,7 +662,14 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
     info->flops = flops;
     return BE_OK;
   }
-  if (!(any_causal && caps) && stream_eligible(dtype, d, g, page_size, flags) && (!caps || caps->tile_rows == 64)) {
+  // causal groups of enough query rows run as 128-row blocks instead
+  const int q_tile = std::max(1, rows_cap / g);
+  int64_t causal_blocks = 0;
+  for (const Group& gr : groups)
+    if (gr.kv_len > 0 && is_causal(gr)) causal_blocks += ceil_div(gr.q1 - gr.q0, q_tile) * hkv;
+  const bool streams = stream_eligible(dtype, d, g, page_size, flags);
+  const bool blocks = streams && !caps && !(flags & BE_PLAN_NO_BLOCKS) && causal_blocks >= kMinCausalBlocks;
+  if (!(any_causal && caps) && streams && !blocks && (!caps || caps->tile_rows == 64)) {
     memset(info, 0, sizeof(*info));
     const int rc = stream_plan(groups, levels, num_levels, total_pages, num_queries, hq, hkv, d, page_size,
                                num_pages, dtype, num_cus, flags, caps, out, cap, info);
@@ -803,7 +688,6 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
     if (rc != BE_ERR_UNSUPPORTED) return rc;
     // a workgroup would need more segments than its table holds: tile kernel
   }
-  const int q_tile = std::max(1, rows_cap / g);
 
   // ---- split-K chunk: about two workgroups per CU over all (tile, chunk, head)
   int64_t work = 0;   // token-tiles
@@ -816,10 +700,44 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   const int64_t chunk_cap = std::max<int64_t>(64, ((int64_t)(kMaxPagesLds - 1) * page_size) / 64 * 64);
   if (chunk > chunk_cap) chunk = chunk_cap;
 
+  // Causal groups on the block kernel: a workgroup's tiles run one after the
+  // other (about 1.5 us each with the CU to itself, 1.05 us per tile of the CU's
+  // two workgroups together: head_dim 128, MI355X), and splitting their keys costs
+  // the merge pass (about 8 us) and the fp32 partials' round trip.  The longest
+  // query tile is cut into the number of chunks, a power of two, that makes the
+  // slower of its own chain and the CUs' shares shortest, those costs included
+  // (1000 fresh tokens, 32 / 8 heads: 32.0 us per layer in two chunks, 28.1
+  // whole).
+  int64_t causal_chunk = 0;
+  if (any_causal && mfma && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
+    int64_t longest = 0, total = 0, queries = 0;
+    for (const Group& gr : groups) {
+      if (gr.kv_len <= 0 || gr.q1 <= gr.q0) continue;
+      queries += gr.q1 - gr.q0;
+      for (int qa = gr.q0; qa < gr.q1; qa += q_tile) {
+        const int64_t t = ceil_div(vis(gr, std::min(qa + q_tile, gr.q1) - 1), kTile);
+        longest = std::max(longest, t);
+        total += t * hkv;
+      }
+    }
+    const double per_d = 0.3 + 0.7 * d / 128;        // a tile's time against head_dim 128
+    double best = 0;
+    for (int64_t cut = 1; cut == 1 || longest / cut >= 8; cut *= 2) {
+      const int64_t c = ceil_div(longest, cut);
+      double t = per_d * std::max(1.5 * c, 1.05 * total / num_cus);
+      if (cut > 1) t += 8.0 + 2.0 * cut * queries * hq * d * 4 / 5e6;
+      if (cut == 1 || t < best) {
+        best = t;
+        causal_chunk = c * kTile;
+      }
+    }
+  }
+
   // A chunk of a group writes rows x D x 4 bytes of partials per KV head while
   // reading 4 x D bytes per token (bf16 K + V): keep chunks >= 4 x rows tokens
   // so partial traffic stays under ~1/4 of the KV bytes it summarises.
   auto group_chunk = [&](const Group& gr) -> int64_t {
+    if (causal_chunk > 0) return std::min(std::max<int64_t>(causal_chunk, kTile), chunk_cap);
     const int64_t rows = (int64_t)std::min(q_tile, gr.q1 - gr.q0) * g;
     int64_t c = std::max<int64_t>(chunk, ceil_div(4 * rows, 64) * 64);
     return std::min(c, chunk_cap);
@@ -868,6 +786,11 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
       }
     }
   }
+
+  // causal items differ in length up to the prompt's: the longest first, so that
+  // the last workgroups to start are the shortest
+  if (any_causal)
+    std::stable_sort(items.begin(), items.end(), [](const WorkItem& x, const WorkItem& y) { return x.tok_count > y.tok_count; });
 
   // ---- merge list (queries with >= 2 partial rows) and zero list (no keys)
   std::vector<int> merge_q, merge_ptr{0}, merge_rows, zero_q;
@@ -949,8 +872,9 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   info->page_size = page_size;
   info->num_pages = num_pages;
   info->dtype = dtype;
-  info->kernel = mfma ? 1 : 0;
-  info->tile_rows = caps ? caps->tile_rows : (max_r <= 16 ? 16 : max_r <= 32 ? 32 : max_r <= 64 ? 64 : 128);
+  info->kernel = blocks ? 2 : mfma ? 1 : 0;
+  info->stream_loop = blocks ? kLoopBlocks : 0;
+  info->tile_rows = blocks ? 128 : caps ? caps->tile_rows : (max_r <= 16 ? 16 : max_r <= 32 ? 32 : max_r <= 64 ? 64 : 128);
   info->chunk_tokens = (int32_t)std::min<int64_t>(chunk, INT32_MAX);
   info->plan_ints = (int32_t)off;
   info->off_items = (int32_t)off_items;
@@ -982,16 +906,15 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
 template <typename T>
 static int launch_attn(const be_attn_plan_info* info, AttnArgs& a, hipStream_t st) {
   const dim3 grid(info->grid_items, info->num_kv_heads);
-  if (info->kernel == 1) {
+  if (info->kernel != 0) {
     if constexpr (sizeof(T) == 2) {
       const int rt = info->tile_rows / 16;
+      if (rt == 8 && block_eligible(info->dtype, info->head_dim)) return block_launch(info, a, st);
 #define BE_TILE_LAUNCH(DD)                                                                    \
   switch (rt) {                                                                               \
     case 1: attn_tile_kernel<T, DD, 1><<<grid, 256, 0, st>>>(a); break;                       \
     case 2: attn_tile_kernel<T, DD, 2><<<grid, 256, 0, st>>>(a); break;                       \
     case 4: attn_tile_kernel<T, DD, 4><<<grid, 256, 0, st>>>(a); break;                       \
-    case 8: if (DD == 256) return fail(BE_ERR_UNSUPPORTED, "128-row tiles at head_dim 256"); \
-            attn_tile_kernel<T, DD, (DD == 256 ? 4 : 8)><<<grid, 256, 0, st>>>(a); break;     \
     default: return fail(BE_ERR_INVALID, "corrupt plan: tile_rows %d", info->tile_rows);      \
   }
       switch (info->head_dim) {
@@ -1038,7 +961,7 @@ int attn_run(const be_attn_plan_info* info, const int32_t* plan, void* partials,
   BE_REQUIRE(info->part_rows_cap == 0 || partials, "plan needs %lld bytes of partial scratch", (long long)info->partial_bytes);
   BE_REQUIRE(info->num_qo_heads % info->num_kv_heads == 0, "corrupt plan info");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (info->kernel == 2)
+  if (info->kernel == 2 && info->stream_loop != kLoopBlocks)
     return stream_run(info, plan, partials, q, q_sn, q_sh, kv, out, o_sn, o_sh, lse, sm_scale, phases, st);
   if (info->kernel == 3) return rows_run(info, plan, q, q_sn, q_sh, kv, out, o_sn, o_sh, lse, sm_scale, phases, st);
   const int64_t rows = info->part_rows_cap;

@@ -167,7 +167,7 @@ typedef struct be_level {
 #define BE_PLAN_CAUSAL 128       /* causal groups on the last level: query q0 + i of a group
                                     of n queries over kv_len tokens sees its first
                                     kv_len - n + i + 1 tokens (FlashInfer's causal prefill
-                                    alignment; such plans run the tile / VALU kernels)     */
+                                    alignment)                                             */
 
 #define BE_PLAN_ROWS 256         /* decode plans: the merge-free row-block kernel (each workgroup
                                     owns up to 16 rows -- queries x GQA heads of one KV head --
@@ -177,6 +177,9 @@ typedef struct be_level {
 #define BE_PLAN_NO_WIDE256 1024  /* streaming kernel: wide roles on 128-row segments only    */
                                  /* (no 256-row segments for groups of >= 256 rows)         */
 #define BE_PLAN_NO_TAIL_ROLE 2048 /* streaming kernel: tail chunks always in the merge kernel */
+#define BE_PLAN_NO_BLOCKS 4096   /* causal groups stay on the streaming kernel where it applies
+                                    (by default plans with many query rows run as 128-row
+                                    blocks, whose split keys take fp32 partial rows)         */
 
 /* Fixed-capacity plan layout (for HIP-graph capture): every region of the
  * device plan sits at an offset that depends only on these capacities, the
@@ -239,7 +242,8 @@ typedef struct be_attn_plan_info {
    * first tail entry, entries, slot) whose results join the records as slots. */
   int32_t num_tail_items;
   int32_t off_tail_items;
-  int32_t stream_loop;     /* streaming kernel's loop: 0 direct global->LDS loads, 1 register-staged */
+  int32_t stream_loop;     /* streaming kernel's loop: 0 direct global->LDS loads, 1 register-staged;
+                              2: causal groups as 128-row blocks (the tile kernels' plan layout) */
   int32_t off_seg_causal;  /* causal plans: per segment, the tokens its first query sees (query j
                               of the segment sees that + j); 0 when the plan has no causal group */
 } be_attn_plan_info;

@@ -607,6 +607,41 @@ def test_causal_flag_without_multi_query_groups_changes_nothing():
     assert np.array_equal(a[2][: a[1].plan_ints], b[2][: b[1].plan_ints])
 
 
+@pytest.mark.parametrize("q_lens,cached,hq,hkv,cus", [([300, 17, 1025], [0, 40, 500], 32, 8, 256), ([256], [8000], 32, 8, 256),
+                                                     ([1100], [3], 8, 8, 256), ([90, 300], [2000, 0], 64, 2, 16)])
+def test_causal_block_plan_covers_visible_tokens(q_lens, cached, hq, hkv, cus):
+    """Causal plans with many query rows take 128-row blocks in the tile kernels'
+    layout: every query's items cover its visible tokens once (the kernel clamps
+    to vis0 + j), the longest first, and BE_PLAN_NO_BLOCKS keeps the streaming
+    plan."""
+    page, qo, kvp, kvi, lpl = 16, [0], [0], [], []
+    for n, c in zip(q_lens, cached):
+        npg = -(-(n + c) // page)
+        kvi += list(range(len(kvi), len(kvi) + npg))
+        kvp.append(len(kvi))
+        lpl.append(n + c - (npg - 1) * page)
+        qo.append(qo[-1] + n)
+    levels = [(qo, kvp, kvi, lpl)]
+    rc, info, buf, _lib, L = plan(levels, hq=hq, hkv=hkv, page=page, num_pages=len(kvi), cus=cus, flags=128)
+    assert rc == 0, L.be_last_error()
+    assert info.kernel == 2 and info.stream_loop == 2 and info.tile_rows == 128
+    items = decode_items(info, buf)
+    assert (items[:, 1] * (hq // hkv) <= 128).all() and (np.diff(items[:, 4]) <= 0).all()
+    seen = [[] for _ in range(qo[-1])]
+    for q0, qn, pb, t0, tc, orow, vis0, _ in items:
+        assert t0 % 64 == 0 and tc > 0
+        for j in range(qn):
+            lim = min(int(tc), max(0, int(vis0) + j - int(t0)))
+            seen[q0 + j].append((int(t0), lim))
+    for r, (n, c) in enumerate(zip(q_lens, cached)):
+        for i in range(n):
+            parts = sorted(seen[qo[r] + i])
+            assert sum(lim for _, lim in parts) == c + i + 1
+            assert all(a + m >= b or m2 == 0 for (a, m), (b, m2) in zip(parts, parts[1:]))
+    rc, info, *_ = plan(levels, hq=hq, hkv=hkv, page=page, num_pages=len(kvi), cus=cus, flags=128 | _lib.BE_PLAN_NO_BLOCKS)
+    assert rc == 0 and (info.kernel, info.stream_loop) != (2, 2)
+
+
 # ---------------------------------------------------------------- row-block plans
 ROWS = 256     # BE_PLAN_ROWS
 

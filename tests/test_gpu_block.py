@@ -1,0 +1,93 @@
+"""128-row block attention (prefill and large groups) on the GPU against the
+float64 oracle, at the edges of its query blocks, token tiles, load groups and
+page windows.  Tolerances are the attention tests' own (16-bit storage: 2e-2
+relative, 1e-2 absolute, against the oracle on the same rounded inputs)."""
+
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as oa
+from tests.test_gpu_prefill import TOL, _check, _levels
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ws():
+    if not torch.cuda.is_available():
+        pytest.skip("no HIP device")
+    return torch.empty(256 << 20, dtype=torch.uint8, device="cuda")
+
+
+def _run(ws, dtype, q_lens, kv_lens, hq, hkv, d, page, causal=True, sm_scale=None, shuffle=3, cus=None):
+    from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
+    (qo, kvp, kvi, lpl), pages = _levels(q_lens, kv_lens, page)
+    g = torch.Generator().manual_seed(shuffle)
+    kvi = torch.randperm(pages, generator=g).tolist()
+    kv = torch.randn((pages, 2, page, hkv, d), generator=g).to(dtype)
+    q = torch.randn((qo[-1], hq, d), generator=g).to(dtype)
+    w = BatchPrefillWithPagedKVCacheWrapper(ws)
+    w._num_cus = cus
+    w.plan(qo, kvp, kvi, lpl, hq, hkv, d, page, causal=causal, sm_scale=sm_scale, q_data_type=dtype)
+    out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
+    torch.cuda.synchronize()
+    ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, sm_scale, causal=causal)
+    _check(out, lse, ref_o, ref_lse, dtype)
+    return w
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("page", [1, 3, 4, 8, 12, 16, 64, 100])
+@pytest.mark.parametrize("d", [64, 128])
+def test_pages_and_head_dims(ws, dtype, page, d):
+    """Page sizes that hold whole load groups (4 rows at head_dim 128, 8 at 64)
+    and ones that do not, prompts around the 32-query block and 64-token tile,
+    with cached tokens before them."""
+    print(f"[case] block page {page} d {d} {dtype}", flush=True)
+    _run(ws, dtype, [33, 129, 64], [33, 200, 65], 16, 4, d, page)
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 8), (12, 4), (40, 8), (64, 2), (48, 1), (128, 1)])
+def test_group_sizes(ws, hq, hkv):
+    """GQA groups that divide the 128-row block and ones that leave rows unused."""
+    print(f"[case] block group {hq}/{hkv}", flush=True)
+    n = 140 if hq // hkv < 32 else 12
+    _run(ws, torch.bfloat16, [n], [n + 77], hq, hkv, 64, 16)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("scale", [0.3, -0.2, 0.0])
+def test_scales_and_unmasked(ws, causal, scale):
+    """Any sign of the scale (the block softmax takes the max of unscaled
+    scores), masked and unmasked."""
+    print(f"[case] block scale {scale} causal {causal}", flush=True)
+    _run(ws, torch.bfloat16, [70, 5], [70, 130], 32, 8, 64, 8, causal=causal, sm_scale=scale)
+
+
+@pytest.mark.parametrize("page", [1, 4, 16])
+def test_keys_split_over_blocks(ws, page):
+    """Few queries over many cached tokens: the keys are cut into chunks (several
+    windows of 64 page ids each) and merged; page 1 also meets the page-id limit
+    of one item."""
+    print(f"[case] block split page {page}", flush=True)
+    w = _run(ws, torch.float16, [40], [3000], 32, 8, 64, page)
+    assert w.stats.num_merge == 40
+
+
+def test_streaming_plan_when_the_workspace_is_too_small():
+    """A causal plan whose fp32 partial rows do not fit the workspace is planned
+    for the streaming kernel, whose 16-bit slots do."""
+    from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
+    (qo, kvp, kvi, lpl), pages = _levels([256], [8256], 16)
+
+    def plan(nbytes):
+        w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(nbytes, dtype=torch.uint8, device="cuda"))
+        w.plan(qo, kvp, kvi, lpl, 32, 8, 128, 16, causal=True, q_data_type=torch.bfloat16)
+        return w
+    full = plan(256 << 20)
+    assert full._info.stream_loop == 2 and full._info.partial_bytes > 0
+    small = plan(full._need(full._info) - 4096)
+    assert small.stats.kernel == "stream" and small._info.stream_loop != 2
