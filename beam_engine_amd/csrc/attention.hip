@@ -33,276 +33,6 @@ struct MergeArgs {
   int hq;
 };
 
-// ================================================================== MFMA kernel
-// bf16/fp16 storage, D in {64, 128, 256}, up to 16*RT rows (queries x GQA
-// group) per workgroup.
-//
-// The workgroup streams its token range in 64-token tiles through LDS: all
-// 256 threads load a tile with 16-byte loads (16 consecutive lanes read one
-// 256-byte K or V row of a page), the next tile's loads are issued before the
-// current tile is computed (register prefetch), and the page ids of the item
-// are staged in LDS once.  K is kept row-major with its 16-byte chunks
-// XOR-swizzled by token; V is stored transposed (head_dim-major) with its
-// tokens XOR-swizzled in groups of four, so the MFMA operand reads are
-// ds_read_b128 / ds_read_b64 with few bank conflicts.
-//
-// Waves own 16-row tiles of the query rows.  With RT <= 2 row tiles the four
-// waves also split the tile's tokens (4/RT ways) and are combined through LDS
-// at the end; with RT >= 4 every wave sees all tokens of its row tiles, so KV
-// is read from HBM once per workgroup however many rows it serves.
-//
-// Scores: S^T = K Q^T with v_mfma_f32_16x16x32 (A = 8 consecutive head_dim
-// elements of a token row, B = Q from registers).  The C layout of a 16-token
-// S^T tile gives lane (lg, lc) tokens 4*lg..4*lg+3 of row lc, which is exactly
-// the B operand (P^T) of v_mfma_f32_16x16x16 for O^T = V^T P^T, whose A
-// operand is 4 consecutive tokens of one head_dim row of the transposed V.
-
-template <int D>
-struct TileLds {
-  static constexpr int CPT = D / 8;                  // 16-byte chunks per token row
-  static constexpr int K_BYTES = kTile * D * 2;
-  static constexpr int V_BYTES = D * kTile * 2;
-};
-
-// V^T token swizzle: groups of four tokens are permuted per 8-row band of head_dim.
-__device__ __forceinline__ int vt_swz(int d) { return (4 * (d >> 3)) & (kTile - 4); }
-
-template <typename T, int D, int RT>
-__global__ __launch_bounds__(256) void attn_tile_kernel(AttnArgs a) {
-  constexpr int KS = D / 32;                         // QK contraction steps
-  constexpr int MT = D / 16;                         // O^T head_dim tiles
-  constexpr int CPT = D / 8;
-  constexpr int LCH = kTile * CPT / 256;             // 16-byte chunks per thread per tile (K and V each)
-  constexpr int NTW = RT <= 4 ? 1 : RT / 4;          // row tiles per wave
-  constexpr int TSPLIT = RT >= 4 ? 1 : 4 / RT;       // waves sharing a row tile (token split)
-  constexpr int STW = (kTile / 16) / TSPLIT;         // 16-token subtiles per wave per tile
-  constexpr int KV_BYTES = TileLds<D>::K_BYTES + TileLds<D>::V_BYTES;
-  constexpr int COMB_SLOT = (MT * 64 * 4 + 2 * 64) * 4;   // bytes: O^T frags + m + l of one wave
-  static_assert(TSPLIT == 1 || (TSPLIT - 1) * RT * COMB_SLOT <= KV_BYTES, "combine scratch must fit");
-  static_assert(LCH >= 1, "tile too small for the workgroup");
-
-  if (a.live_items && (int)blockIdx.x >= *a.live_items) return;
-  __shared__ __attribute__((aligned(16))) unsigned char kv_lds[KV_BYTES];
-  __shared__ int pg_lds[kMaxPagesLds];
-  uint16_t* kt = reinterpret_cast<uint16_t*>(kv_lds);
-  uint16_t* vt = reinterpret_cast<uint16_t*>(kv_lds + TileLds<D>::K_BYTES);
-
-  const WorkItem it = a.items[blockIdx.x];
-  const int kvh = blockIdx.y;
-  const int tid = threadIdx.x;
-  const int w = tid >> 6, lane = tid & 63, lg = lane >> 4, lc = lane & 15;
-  const int g = a.g, R = it.q_count * g, ps = a.page_size;
-  const T* kv = reinterpret_cast<const T*>(a.kv);
-
-  // ---- page ids of the item
-  const int first_page = it.tok_begin / ps;
-  const int n_pages = (it.tok_begin + it.tok_count - 1) / ps - first_page + 1;
-  for (int i = tid; i < n_pages; i += 256) pg_lds[i] = a.pages[it.page_begin + first_page + i];
-
-  // ---- wave role
-  const int rt0 = (RT >= 4) ? w * NTW : (w % RT);
-  const int ts = (RT >= 4) ? 0 : (w / RT);
-  bool active[NTW];
-  int lim[NTW];      // item tokens this lane's row sees (causal: its query's limit)
-#pragma unroll
-  for (int nt = 0; nt < NTW; ++nt) {
-    active[nt] = (rt0 + nt) * 16 < R;
-    const int64_t v = (int64_t)it.vis0 + ((rt0 + nt) * 16 + lc) / g - it.tok_begin;
-    lim[nt] = (int)std::min<int64_t>(it.tok_count, std::max<int64_t>(v, 0));
-  }
-
-  // ---- Q as the B operand: lane holds Q[row = (rt0+nt)*16 + lc][d = ks*32 + 8*lg .. +7]
-  v8s qf[NTW][KS];
-#pragma unroll
-  for (int nt = 0; nt < NTW; ++nt) {
-    const int row = (rt0 + nt) * 16 + lc;
-    if (row < R) {
-      const int j = row / g, hh = row - j * g;
-      const int qi = a.q_index[it.q_begin + j];
-      const T* qp = reinterpret_cast<const T*>(a.q) + (int64_t)qi * a.q_sn + (int64_t)(kvh * g + hh) * a.q_sh;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qf[nt][ks] = *reinterpret_cast<const v8s*>(qp + ks * 32 + lg * 8);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qf[nt][ks] = v8s{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-  }
-  __syncthreads();   // page ids staged
-
-  // ---- tile loader: thread chunk c = i*256 + tid -> token c / CPT, column chunk c % CPT
-  v8s kp[LCH], vp[LCH];
-  auto load_tile = [&](int tile) {
-#pragma unroll
-    for (int i = 0; i < LCH; ++i) {
-      const int c = i * 256 + tid;
-      const int tl = tile * kTile + c / CPT;
-      if (tl < it.tok_count) {
-        const int tok = it.tok_begin + tl;
-        const int page = pg_lds[tok / ps - first_page];
-        const int64_t base = kv_off(page, 0, tok % ps, kvh, ps, a.hkv, D) + (c % CPT) * 8;
-        const int64_t vstep = (int64_t)ps * a.hkv * D;     // K plane -> V plane of the page
-        kp[i] = *reinterpret_cast<const v8s*>(kv + base);
-        vp[i] = *reinterpret_cast<const v8s*>(kv + base + vstep);
-      } else {
-        kp[i] = v8s{0, 0, 0, 0, 0, 0, 0, 0};
-        vp[i] = v8s{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
-  };
-
-  float m_run[NTW], l_run[NTW];
-  v4f o_acc[NTW][MT];
-#pragma unroll
-  for (int nt = 0; nt < NTW; ++nt) {
-    m_run[nt] = -INFINITY;
-    l_run[nt] = 0.f;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) o_acc[nt][mt] = v4f{0.f, 0.f, 0.f, 0.f};
-  }
-
-  const int n_tiles = (it.tok_count + kTile - 1) / kTile;
-  load_tile(0);
-  for (int tile = 0; tile < n_tiles; ++tile) {
-    __syncthreads();                                   // previous tile's LDS reads are done
-#pragma unroll
-    for (int i = 0; i < LCH; ++i) {
-      const int c = i * 256 + tid;
-      const int t = c / CPT, ch = c % CPT;
-      *reinterpret_cast<v8s*>(kt + (t * CPT + (ch ^ (t & (CPT - 1)))) * 8) = kp[i];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = ch * 8 + e;
-        vt[d * kTile + (t ^ vt_swz(d))] = (uint16_t)vp[i][e];
-      }
-    }
-    __syncthreads();                                   // tile staged
-    if (tile + 1 < n_tiles) load_tile(tile + 1);       // in flight during the compute below
-
-    const int tl0 = tile * kTile;
-#pragma unroll
-    for (int nt = 0; nt < NTW; ++nt) {
-      if (!active[nt]) continue;
-      // scores of the wave's subtiles (lane: tokens 16*sub + 4*lg + r, row lc)
-      float x[STW][4];
-#pragma unroll
-      for (int sb = 0; sb < STW; ++sb) {
-        const int sub = ts * STW + sb;
-        const int t = sub * 16 + lc;
-        v4f acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const int ch = ks * 4 + lg;
-          const v8s kf = *reinterpret_cast<const v8s*>(kt + (t * CPT + (ch ^ (t & (CPT - 1)))) * 8);
-          acc = mfma_qk<T>(kf, qf[nt][ks], acc);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int tl = tl0 + sub * 16 + 4 * lg + r;
-          x[sb][r] = (tl < lim[nt]) ? acc[r] * a.scale_log2 : -INFINITY;
-        }
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int sb = 0; sb < STW; ++sb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) mx = fmaxf(mx, x[sb][r]);
-      mx = rows4_max(mx);
-      const float m_new = fmaxf(m_run[nt], mx);
-      const float msafe = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = exp2f(m_run[nt] - msafe);    // 0 while nothing was seen
-      float psum = 0.f;
-      v4s pf[STW];
-#pragma unroll
-      for (int sb = 0; sb < STW; ++sb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float p = exp2f(x[sb][r] - msafe);
-          psum += p;
-          pf[sb][r] = (short)pack16<T>(p);
-        }
-      l_run[nt] = l_run[nt] * alpha + psum;
-      m_run[nt] = m_new;
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        v4f o = o_acc[nt][mt] * alpha;
-#pragma unroll
-        for (int sb = 0; sb < STW; ++sb) {
-          const int d = mt * 16 + lc;
-          const int tok = (ts * STW + sb) * 16 + 4 * lg;
-          const v4s vf = *reinterpret_cast<const v4s*>(vt + d * kTile + (tok ^ vt_swz(d)));
-          o = mfma_pv<T>(vf, pf[sb], o);
-        }
-        o_acc[nt][mt] = o;
-      }
-    }
-  }
-
-  // row sums over the four lane groups
-#pragma unroll
-  for (int nt = 0; nt < NTW; ++nt) {
-    l_run[nt] = rows4_sum(l_run[nt]);
-  }
-
-  // ---- token-split waves (ts > 0) hand their state to the ts == 0 wave of the row tile
-  if constexpr (TSPLIT > 1) {
-    float* comb = reinterpret_cast<float*>(kv_lds);
-    __syncthreads();                                   // tiles no longer needed
-    if (ts > 0 && active[0]) {
-      float* slot = comb + ((ts - 1) * RT + rt0) * (COMB_SLOT / 4);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<v4f*>(slot + (mt * 64 + lane) * 4) = o_acc[0][mt];
-      slot[MT * 256 + lane] = m_run[0];
-      slot[MT * 256 + 64 + lane] = l_run[0];
-    }
-    __syncthreads();
-    if (ts == 0 && active[0]) {
-#pragma unroll
-      for (int s2 = 1; s2 < TSPLIT; ++s2) {
-        const float* slot = comb + ((s2 - 1) * RT + rt0) * (COMB_SLOT / 4);
-        const float mb = slot[MT * 256 + lane], lb = slot[MT * 256 + 64 + lane];
-        const float M = fmaxf(m_run[0], mb);
-        const float ca = (M == -INFINITY) ? 0.f : exp2f(m_run[0] - M);
-        const float cb = (M == -INFINITY) ? 0.f : exp2f(mb - M);
-        l_run[0] = l_run[0] * ca + lb * cb;
-        m_run[0] = M;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-          o_acc[0][mt] = o_acc[0][mt] * ca + *reinterpret_cast<const v4f*>(slot + (mt * 64 + lane) * 4) * cb;
-      }
-    }
-  }
-
-  // ---- writes: lane holds O^T[d = mt*16 + 4*lg + i][row = (rt0+nt)*16 + lc]
-  if (ts == 0) {
-#pragma unroll
-    for (int nt = 0; nt < NTW; ++nt) {
-      const int row = (rt0 + nt) * 16 + lc;
-      if (!active[nt] || row >= R) continue;
-      const int j = row / g, hh = row - j * g, head = kvh * g + hh;
-      const float l = l_run[nt];
-      const float inv = (l > 0.f) ? 1.f / l : 0.f;
-      if (it.out_row < 0) {
-        const int qi = a.q_index[it.q_begin + j];
-        T* op = reinterpret_cast<T*>(a.out) + (int64_t)qi * a.o_sn + (int64_t)head * a.o_sh;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          v4s pk;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) pk[i] = (short)pack16<T>(o_acc[nt][mt][i] * inv);
-          *reinterpret_cast<v4s*>(op + mt * 16 + 4 * lg) = pk;
-        }
-      } else {
-        float* op = a.part_o + ((int64_t)(it.out_row + j) * a.hq + head) * D;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) *reinterpret_cast<v4f*>(op + mt * 16 + 4 * lg) = o_acc[nt][mt] * inv;
-      }
-      if (lg == 0) store_row_lse<T>(a, it, j, head, m_run[nt], l);
-    }
-  }
-  __shared__ int s_last[kMaxTileRows];
-  if (it.out_row >= 0 && a.counters) fused_merge_epilogue<T, D>(a, it, kvh, s_last);
-}
-
 // ================================================================== VALU kernel
 // Any storage dtype, D in {64, 128, 256}, up to 32 rows per tile.  K/V blocks
 // of 32 tokens are converted to fp32 in LDS; scores use one thread per
@@ -430,80 +160,56 @@ __global__ __launch_bounds__(256) void attn_valu_kernel(AttnArgs a) {
 }
 
 // ================================================================== merge kernel
-// One workgroup per merged query: the lse of every (partial row, head) pair is
-// read in parallel and turned into normalised weights in LDS, then every
-// thread accumulates 4 consecutive head_dim columns of one head over the rows
-// (independent loads, no dependent chain).
-constexpr int kMergeMaxRows = 64;
+// One thread per (merged query, head, 4 head_dim columns): eight partial rows'
+// lse and o at a time (their loads issued together), combined by log-sum-exp
+// with a running max.  No LDS and no barrier: the launch is a chain of dependent
+// round trips (row range, row ids, lse and o) and little else, so the heads of a
+// query are spread over workgroups.  One workgroup per query with the weights in
+// LDS took 9.8 us for 32 queries of 17 partial rows (32 heads, head_dim 64,
+// MI355X), 5.6 us now; 8 queries of 4 rows (head_dim 128) 5.3 -> 3.2 us.
+constexpr int kMergeBatch = 8;
 
 template <typename T, int D>
 __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
-  __shared__ float wgt[kMergeMaxRows * kMaxTileRows];   // [row][head] weights
-  __shared__ int rows_s[kMergeMaxRows];
-  __shared__ float lse_h[kMaxTileRows];
+  constexpr int C4 = D / 4;                       // float4 columns per head
   if (a.live && (int)blockIdx.x >= *a.live) return;
-  const int tid = threadIdx.x;
+  const int i = blockIdx.y * 256 + threadIdx.x, h = i / C4, c = i - h * C4;
+  const int hq = a.hq;
+  if (h >= hq) return;
   const int qi = a.merge_q[blockIdx.x];
   const int b = a.merge_ptr[blockIdx.x], e = a.merge_ptr[blockIdx.x + 1];
-  const int hq = a.hq;
-  T* out = reinterpret_cast<T*>(a.out) + (int64_t)qi * a.o_sn;
-  if (e - b > kMergeMaxRows || hq > kMaxTileRows) {
-    // long merges: one wave per head, sequential over rows
-    for (int head = tid >> 6; head < hq; head += 4) {
-      const int lane = tid & 63;
-      float M = -INFINITY;
-      for (int i = b; i < e; ++i) M = fmaxf(M, a.part_lse[(int64_t)a.merge_rows[i] * hq + head]);
-      float z = 0.f, acc[D / 64];
+  float M = -INFINITY, z = 0.f;
+  v4f acc = {0.f, 0.f, 0.f, 0.f};
+  for (int r0 = b; r0 < e; r0 += kMergeBatch) {
+    float l[kMergeBatch];
+    v4f o[kMergeBatch];
 #pragma unroll
-      for (int k = 0; k < D / 64; ++k) acc[k] = 0.f;
-      if (M != -INFINITY)
-        for (int i = b; i < e; ++i) {
-          const int64_t row = (int64_t)a.merge_rows[i] * hq + head;
-          const float w = expf(a.part_lse[row] - M);
-          z += w;
-#pragma unroll
-          for (int k = 0; k < D / 64; ++k) acc[k] += w * a.part_o[row * D + lane + 64 * k];
-        }
-      const float inv = (z > 0.f) ? 1.f / z : 0.f;
-#pragma unroll
-      for (int k = 0; k < D / 64; ++k) out[(int64_t)head * a.o_sh + lane + 64 * k] = from_f32<T>(acc[k] * inv);
-      if (a.out_lse && lane == 0) a.out_lse[(int64_t)qi * hq + head] = (z > 0.f) ? M + logf(z) : -INFINITY;
+    for (int u = 0; u < kMergeBatch; ++u) {
+      const int64_t row = (int64_t)a.merge_rows[min(r0 + u, e - 1)] * hq + h;
+      l[u] = r0 + u < e ? a.part_lse[row] : -INFINITY;
+      o[u] = *reinterpret_cast<const v4f*>(a.part_o + row * D + 4 * c);
     }
-    return;
-  }
-  const int nr = e - b;
-  for (int i = tid; i < nr; i += 256) rows_s[i] = a.merge_rows[b + i];
-  __syncthreads();
-  for (int i = tid; i < nr * hq; i += 256) {
-    const int r = i / hq, h = i - r * hq;
-    wgt[r * hq + h] = a.part_lse[(int64_t)rows_s[r] * hq + h];
-  }
-  __syncthreads();
-  for (int h = tid; h < hq; h += 256) {
-    float M = -INFINITY;
-    for (int r = 0; r < nr; ++r) M = fmaxf(M, wgt[r * hq + h]);
-    float z = 0.f;
-    if (M != -INFINITY)
-      for (int r = 0; r < nr; ++r) z += expf(wgt[r * hq + h] - M);
-    const float inv = (z > 0.f) ? 1.f / z : 0.f;
-    for (int r = 0; r < nr; ++r) wgt[r * hq + h] = (M != -INFINITY) ? expf(wgt[r * hq + h] - M) * inv : 0.f;
-    lse_h[h] = (z > 0.f) ? M + logf(z) : -INFINITY;
-  }
-  __syncthreads();
-  constexpr int C4 = D / 4;                       // float4 columns per head
-  for (int i = tid; i < hq * C4; i += 256) {
-    const int h = i / C4, c = i - h * C4;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    for (int r = 0; r < nr; ++r) {
-      const v4f o = *reinterpret_cast<const v4f*>(a.part_o + ((int64_t)rows_s[r] * hq + h) * D + 4 * c);
-      acc += o * wgt[r * hq + h];
-    }
-    T* op = out + (int64_t)h * a.o_sh + 4 * c;
+    float m = M;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) op[k] = from_f32<T>(acc[k]);
+    for (int u = 0; u < kMergeBatch; ++u) m = fmaxf(m, l[u]);
+    if (m == -INFINITY) continue;                 // nothing seen yet
+    const float s = expf(M - m);
+    z *= s;
+    acc *= s;
+#pragma unroll
+    for (int u = 0; u < kMergeBatch; ++u) {
+      const float wgt = expf(l[u] - m);
+      z += wgt;
+      // (a row past the end or one that saw no key holds no finite o to add)
+      if (l[u] != -INFINITY) acc += o[u] * wgt;
+    }
+    M = m;
   }
-  if (a.out_lse)
-    for (int h = tid; h < hq; h += 256) a.out_lse[(int64_t)qi * hq + h] = lse_h[h];
+  const float inv = (z > 0.f) ? 1.f / z : 0.f;
+  T* op = reinterpret_cast<T*>(a.out) + (int64_t)qi * a.o_sn + (int64_t)h * a.o_sh + 4 * c;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) op[k] = from_f32<T>(acc[k] * inv);
+  if (a.out_lse && c == 0) a.out_lse[(int64_t)qi * hq + h] = (z > 0.f) ? M + logf(z) : -INFINITY;
 }
 
 // One wave owns one row, so outputs may alias inputs (every lane reads the
@@ -907,26 +613,9 @@ template <typename T>
 static int launch_attn(const be_attn_plan_info* info, AttnArgs& a, hipStream_t st) {
   const dim3 grid(info->grid_items, info->num_kv_heads);
   if (info->kernel != 0) {
-    if constexpr (sizeof(T) == 2) {
-      const int rt = info->tile_rows / 16;
-      if (rt == 8 && block_eligible(info->dtype, info->head_dim)) return block_launch(info, a, st);
-#define BE_TILE_LAUNCH(DD)                                                                    \
-  switch (rt) {                                                                               \
-    case 1: attn_tile_kernel<T, DD, 1><<<grid, 256, 0, st>>>(a); break;                       \
-    case 2: attn_tile_kernel<T, DD, 2><<<grid, 256, 0, st>>>(a); break;                       \
-    case 4: attn_tile_kernel<T, DD, 4><<<grid, 256, 0, st>>>(a); break;                       \
-    default: return fail(BE_ERR_INVALID, "corrupt plan: tile_rows %d", info->tile_rows);      \
-  }
-      switch (info->head_dim) {
-        case 64: BE_TILE_LAUNCH(64) break;
-        case 128: BE_TILE_LAUNCH(128) break;
-        case 256: BE_TILE_LAUNCH(256) break;
-        default: return fail(BE_ERR_UNSUPPORTED, "head_dim %d", info->head_dim);
-      }
-#undef BE_TILE_LAUNCH
-    } else {
-      return fail(BE_ERR_UNSUPPORTED, "MFMA kernel needs fp16/bf16 storage");
-    }
+    if (info->dtype == BE_F32) return fail(BE_ERR_UNSUPPORTED, "MFMA kernel needs fp16/bf16 storage");
+    if (info->tile_rows == kMaxTileRows && block_eligible(info->dtype, info->head_dim)) return block_launch(info, a, st);
+    return tile_launch(info, a, st);
   } else {
     switch (info->head_dim) {
       case 64: attn_valu_kernel<T, 64><<<grid, 256, 0, st>>>(a); break;
@@ -941,7 +630,7 @@ static int launch_attn(const be_attn_plan_info* info, AttnArgs& a, hipStream_t s
 
 template <typename T>
 static int launch_merge(const be_attn_plan_info* info, MergeArgs& m, int count, hipStream_t st) {
-  const dim3 grid(count);
+  const dim3 grid(count, (info->num_qo_heads * (info->head_dim / 4) + 255) / 256);
   switch (info->head_dim) {
     case 64: merge_kernel<T, 64><<<grid, 256, 0, st>>>(m); break;
     case 128: merge_kernel<T, 128><<<grid, 256, 0, st>>>(m); break;

@@ -31,13 +31,10 @@
 #include <math.h>
 
 #include "attn_tile.h"
-#include "stream_device.h"
 
 namespace be {
 namespace block {
 
-using stream::dma16;
-using stream::dma16_sv;
 using stream::lds_addr;
 using stream::lds_v4s_t;
 using stream::pack2;
@@ -89,23 +86,16 @@ __device__ __forceinline__ float other_half_sum(float x) {
 // 16-bit P and the fp32 sums, with the same relative rounding.
 constexpr float kLag = 8.f;
 
-// PAGED4: pages hold whole load instructions' rows (4 tokens at head_dim 128, 8
-// at 64), so a load's page is wave-uniform: its id comes from a register by
-// v_readlane, the address is scalar and a tile's loads cost no vector
-// arithmetic.  Otherwise every lane looks its row's page up in LDS.
 template <typename T, int D, bool PAGED4>
 __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_items) {
   constexpr int KS = D / 16;                         // QK contraction steps
   constexpr int MB = D / 32;                         // Oᵀ head_dim blocks
   constexpr int RB = D * 2;                          // bytes of a K or V row
-  constexpr int CPR = RB / 16;                       // 16-byte chunks per row
-  constexpr int RPI = 64 / CPR;                      // rows per wave load instruction
-  constexpr int IPW = kTile / RPI / 4;               // load instructions per wave per tile (K and V each)
-  constexpr int PLANE = kTile * RB;                  // bytes of a K or V tile
-  constexpr int STAGE = 2 * PLANE;
+  using Loader = TileLoader<RB, PAGED4, swz<D>>;
+  constexpr int CPR = Loader::CPR, RPI = Loader::RPI, PLANE = Loader::PLANE, STAGE = Loader::STAGE;
 
   __shared__ __attribute__((aligned(1024))) unsigned char stage[2 * STAGE];
-  __shared__ uint32_t pg_lds[kMaxPagesLds];
+  __shared__ int32_t pg_lds[kMaxPagesLds];
   // consecutive workgroups are the KV heads of one item: with 8 (or a divisor)
   // heads an XCD keeps the same heads' K and V in its L2
   const int item = (int)blockIdx.x / a.hkv, kvh = (int)blockIdx.x - item * a.hkv;
@@ -120,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
   // ---- the item's pages
   const int first_page = it.tok_begin / ps;
   const int n_pages = (it.tok_begin + it.tok_count - 1) / ps - first_page + 1;
-  for (int i = tid; i < n_pages; i += 256) pg_lds[i] = (uint32_t)a.pages[it.page_begin + first_page + i];
+  for (int i = tid; i < n_pages; i += 256) pg_lds[i] = a.pages[it.page_begin + first_page + i];
 
   // ---- this wave's rows: lane's row, the tokens it sees, the wave's most
   const int row = w * kWaveRows + lr;
@@ -154,74 +144,11 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = v8s{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  __syncthreads();                                   // page ids staged
-
-  // ---- tile loader: instruction i of wave w moves rows (w IPW + i) RPI .. + RPI - 1
-  // of K and of V; the lane's LDS chunk lane % CPR holds the row's chunk
-  // (lane % CPR) ^ swz(row).  Rows past the item's end re-read its last token
-  // (masked).  Pages and slots advance by whole tiles without a division.
+  if constexpr (!PAGED4) __syncthreads();            // page ids staged (else by the first tile's barrier)
+  Loader ld;
+  ld.init(a, it, kvh, w, pg_lds, first_page, n_pages);
   const uint32_t lds0 = lds_addr(stage);
-  const uint32_t row_bytes = (uint32_t)a.hkv * RB;
-  const uint64_t vplane = (uint64_t)ps * row_bytes;
-  const int dpage = kTile / ps, dslot = kTile % ps;
-  const int last_page = n_pages - 1, last_slot = (it.tok_begin + it.tok_count - 1) % ps;
-  const uint64_t kvb = reinterpret_cast<uint64_t>(a.kv) + (uint64_t)kvh * RB;
-  const int lrow4 = lane / CPR;                      // the lane's row within a load
-  int ld_page[IPW], ld_slot[IPW];                    // (wave-uniform if PAGED4)
-  uint32_t ld_off[IPW];
-#pragma unroll
-  for (int i = 0; i < IPW; ++i) {
-    const int r0 = (w * IPW + i) * RPI, r = r0 + (PAGED4 ? 0 : lrow4);
-    ld_page[i] = (it.tok_begin + r) / ps - first_page;
-    ld_slot[i] = (it.tok_begin + r) % ps;
-    ld_off[i] = ((lane % CPR) ^ swz<D>(r0 + lrow4)) << 4;
-  }
-  int ld_tok = 0, pg_base = 0;                       // first token of the next tile; page index of lane 0's id
-  int pg_reg = PAGED4 ? (int)pg_lds[min(lane, n_pages - 1)] : 0;
-  auto load_tile = [&](int st) {
-    if constexpr (PAGED4) {
-      // the tile's pages lie within 64 of its first (a page holds at least RPI tokens)
-      const int p0 = min(ld_page[0], last_page), p1 = min(ld_page[IPW - 1], last_page);
-      if (p1 - pg_base >= 64) {
-        pg_base = p0;
-        pg_reg = (int)pg_lds[min(pg_base + lane, n_pages - 1)];
-      }
-    }
-    const bool whole = ld_tok + kTile <= it.tok_count;   // uniform
-#pragma unroll
-    for (int i = 0; i < IPW; ++i) {
-      const int r0 = (w * IPW + i) * RPI;
-      const uint32_t dst = lds0 + st * STAGE + (w * IPW + i) * 1024;
-      if constexpr (PAGED4) {
-        int page = ld_page[i], slot = ld_slot[i], lr4 = lrow4;
-        if (!whole) {
-          const int left = it.tok_count - 1 - (ld_tok + r0);   // rows of this load up to the last token
-          if (left < 0) {
-            page = last_page;
-            slot = last_slot;
-          }
-          lr4 = min(lrow4, max(left, 0));
-        }
-        const int id = __builtin_amdgcn_readlane(pg_reg, page - pg_base);
-        const uint64_t base = kvb + (uint64_t)((uint32_t)id * 2u * (uint32_t)ps + (uint32_t)slot) * row_bytes;
-        const uint32_t off = (uint32_t)lr4 * row_bytes + ld_off[i];
-        dma16_sv(base, off, dst);
-        dma16_sv(base + vplane, off, dst + PLANE);
-      } else {
-        const bool in = whole || ld_tok + r0 + lrow4 < it.tok_count;
-        const uint32_t rec = pg_lds[in ? ld_page[i] : last_page] * 2u * (uint32_t)ps + (uint32_t)(in ? ld_slot[i] : last_slot);
-        const uint64_t src = kvb + ld_off[i] + (uint64_t)rec * row_bytes;
-        dma16(reinterpret_cast<const void*>(src), dst);
-        dma16(reinterpret_cast<const void*>(src + vplane), dst + PLANE);
-      }
-      ld_slot[i] += dslot;
-      const bool carry = ld_slot[i] >= ps;
-      ld_slot[i] -= carry ? ps : 0;
-      ld_page[i] += dpage + (carry ? 1 : 0);
-    }
-    ld_tok += kTile;
-  };
-  load_tile(0);
+  ld.load(lds0);
   // Q has landed before the loop: the compiler would otherwise wait for it, and
   // with it for the tile loads issued since, in every iteration
 #pragma unroll
@@ -253,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
     // this wave's loads of the tile have landed; after the barrier everyone's
     // have, and everyone is done with the other stage
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (tile + 1 < n_tiles) load_tile(st ^ 1);
+    if (tile + 1 < n_tiles) ld.load(lds0 + (st ^ 1) * STAGE);
     const int t0 = tile * kTile;
     if (!wave_on || t0 >= lim_most) continue;
     const unsigned char* kt = stage + st * STAGE;
@@ -386,7 +313,7 @@ bool block_eligible(int dtype, int head_dim) {
 int block_launch(const be_attn_plan_info* info, const AttnArgs& a, hipStream_t st) {
   const int n = info->grid_items;
   const unsigned blocks = (unsigned)n * (unsigned)info->num_kv_heads;
-  const bool p4 = info->page_size % (info->head_dim == 128 ? 4 : 8) == 0;
+  const bool p4 = paged4(info->page_size, info->head_dim * 2);
 #define BE_BLOCK_LAUNCH(TY, DD)                                                        \
   if (p4) block::attn_block_kernel<TY, DD, true><<<blocks, 256, 0, st>>>(a, n);         \
   else block::attn_block_kernel<TY, DD, false><<<blocks, 256, 0, st>>>(a, n);

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "attention.h"
+#include "stream_device.h"
 
 namespace be {
 
@@ -128,6 +129,113 @@ __device__ void fused_merge_epilogue(const AttnArgs& a, const WorkItem& it, int 
     if (tid == 0) a.counters[(int64_t)mi * a.hkv + kvh] = 0;
   }
 }
+
+// ---------------------------------------------------------------- tile loads
+// K and V rows of an item, 64 tokens at a time, global -> LDS directly by the
+// four waves of a workgroup: K at the stage's start, V one plane further, rows of
+// RB bytes whose 16-byte chunk c sits at slot c ^ swz(row).  Load i of wave w
+// moves rows (w IPW + i) RPI .. + RPI - 1 (1 KB of K and 1 KB of V); rows past
+// the item's end re-read its last token (the caller masks them).  Pages and slots
+// advance by whole tiles without a division.
+//
+// PAGED4: pages hold whole loads' rows (1 KB: 4 tokens of 256-byte rows), so a load's page is wave-uniform: its id comes from a register (64 of the
+// item's ids) by v_readlane, the address is scalar, and a tile's loads cost no
+// vector arithmetic.  Otherwise every lane looks its row's page up in pg_lds
+// (the caller stages the item's page ids there and synchronises first).
+template <int RB, bool PAGED4, int (*SWZ)(int)>
+struct TileLoader {
+  static constexpr int CPR = RB / 16;                  // 16-byte chunks per row
+  static constexpr int RPI = 64 / CPR;                 // rows per wave load
+  static constexpr int IPW = kTile / RPI / 4;          // loads per wave per tile (K and V each)
+  static constexpr int PLANE = kTile * RB;
+  static constexpr int STAGE = 2 * PLANE;
+
+  uint64_t kvb, vplane;
+  uint32_t row_bytes, off[IPW];
+  int w, lane, ps, tok_count, dpage, dslot, last_page, last_slot;
+  int page[IPW], slot[IPW];                            // of the next tile's loads (wave-uniform if PAGED4)
+  int tok, pg_base, pg_reg;                            // next tile's first token; the register's first page
+  const int32_t* pg_lds;
+
+  __device__ __forceinline__ void init(const AttnArgs& a, const WorkItem& it, int kvh, int wave, const int32_t* lds,
+                                       int first_page, int n_pages) {
+    w = wave;
+    lane = threadIdx.x & 63;
+    ps = a.page_size;
+    tok_count = it.tok_count;
+    pg_lds = lds;
+    row_bytes = (uint32_t)a.hkv * RB;
+    vplane = (uint64_t)ps * row_bytes;
+    kvb = reinterpret_cast<uint64_t>(a.kv) + (uint64_t)kvh * RB;
+    dpage = kTile / ps;
+    dslot = kTile % ps;
+    last_page = n_pages - 1;
+    last_slot = (it.tok_begin + it.tok_count - 1) % ps;
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) {
+      const int r0 = (w * IPW + i) * RPI, r = r0 + (PAGED4 ? 0 : lane / CPR);
+      page[i] = (it.tok_begin + r) / ps - first_page;
+      slot[i] = (it.tok_begin + r) % ps;
+      off[i] = ((lane % CPR) ^ SWZ(r0 + lane / CPR)) << 4;
+    }
+    tok = 0;
+    pg_base = 0;
+    // (the first 64 ids from memory: no barrier before the first loads)
+    pg_reg = PAGED4 ? a.pages[it.page_begin + first_page + min(lane, last_page)] : 0;
+  }
+
+  // The next tile's loads, to LDS byte address dst0 (2 IPW vector memory operations).
+  __device__ __forceinline__ void load(uint32_t dst0) {
+    if constexpr (PAGED4) {
+      // the wave's rows of a tile lie within 64 pages of its first (a page holds at least RPI tokens)
+      const int p1 = min(page[IPW - 1], last_page);
+      if (p1 - pg_base >= 64) {
+        pg_base = min(page[0], last_page);
+        pg_reg = pg_lds[min(pg_base + lane, last_page)];
+      }
+    }
+    const bool whole = tok + kTile <= tok_count;         // uniform
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) {
+      const int r0 = (w * IPW + i) * RPI;
+      const uint32_t dst = dst0 + (w * IPW + i) * 1024;
+      if constexpr (PAGED4) {
+        int pg = page[i], sl = slot[i], lr = lane / CPR;
+        if (!whole) {
+          const int left = tok_count - 1 - (tok + r0);   // rows of this load up to the last token
+          if (left < 0) {
+            pg = last_page;
+            sl = last_slot;
+          }
+          lr = min(lr, max(left, 0));
+        }
+        const int id = __builtin_amdgcn_readlane(pg_reg, pg - pg_base);
+        const uint64_t base = kvb + (uint64_t)((uint32_t)id * 2u * (uint32_t)ps + (uint32_t)sl) * row_bytes;
+        const uint32_t o = (uint32_t)lr * row_bytes + off[i];
+        stream::dma16_sv(base, o, dst);
+        stream::dma16_sv(base + vplane, o, dst + PLANE);
+      } else {
+        const bool in = whole || tok + r0 + lane / CPR < tok_count;
+        const uint32_t rec = (uint32_t)pg_lds[in ? page[i] : last_page] * 2u * (uint32_t)ps + (uint32_t)(in ? slot[i] : last_slot);
+        const uint64_t src = kvb + off[i] + (uint64_t)rec * row_bytes;
+        stream::dma16(reinterpret_cast<const void*>(src), dst);
+        stream::dma16(reinterpret_cast<const void*>(src + vplane), dst + PLANE);
+      }
+      slot[i] += dslot;
+      const bool carry = slot[i] >= ps;
+      slot[i] -= carry ? ps : 0;
+      page[i] += dpage + (carry ? 1 : 0);
+    }
+    tok += kTile;
+  }
+};
+
+// Whether pages of this size hold whole loads of rows of this many bytes.
+inline bool paged4(int page_size, int row_bytes) { return page_size % (1024 / row_bytes) == 0; }
+
+// Launches the 16-row-tile kernel (attn_tile.hip) over a work list whose items
+// hold up to 64 rows: one workgroup per (item, KV head).
+int tile_launch(const be_attn_plan_info* info, const AttnArgs& a, hipStream_t st);
 
 // ---------------------------------------------------------------- 128-row blocks (attn_block.hip)
 // A streaming plan's stream_loop when its causal groups run as 128-row blocks.

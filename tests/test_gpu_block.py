@@ -67,6 +67,18 @@ def test_scales_and_unmasked(ws, causal, scale):
     _run(ws, torch.bfloat16, [70, 5], [70, 130], 32, 8, 64, 8, causal=causal, sm_scale=scale)
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("page", [1, 2, 3, 8, 16])
+@pytest.mark.parametrize("rows", [(4, 1), (3, 4), (5, 8), (1, 40)])
+def test_few_rows(ws, d, page, rows):
+    """Items of one to four 16-row tiles (the waves split the tokens of few rows
+    and are combined), token counts around one and two tiles and beyond 64 page
+    ids, causal, at every head_dim."""
+    n, g = rows
+    print(f"[case] tile rows {n} x {g} d {d} page {page}", flush=True)
+    _run(ws, torch.bfloat16, [n, n, n], [63, 130, 400], 2 * g, 2, d, page)
+
+
 @pytest.mark.parametrize("page", [1, 4, 16])
 def test_keys_split_over_blocks(ws, page):
     """Few queries over many cached tokens: the keys are cut into chunks (several
