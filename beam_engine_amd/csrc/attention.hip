@@ -333,8 +333,10 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   bool mfma = (dtype != BE_F32) && !(flags & BE_PLAN_FORCE_VALU);
   if (!mfma && g > kMaxRows) return fail(BE_ERR_UNSUPPORTED, "GQA group %d exceeds %d (VALU kernel)", g, kMaxRows);
   if (mfma && d == 256 && g > 64) return fail(BE_ERR_UNSUPPORTED, "GQA group %d exceeds 64 at head_dim 256", g);
-  // rows per workgroup: MFMA 8 row tiles (4 at head_dim 256, VGPR budget), VALU 32
-  int rows_cap = mfma ? (d == 256 ? 64 : kMaxTileRows) : kMaxRows;
+  // rows per workgroup: MFMA 8 row tiles (4 at head_dim 256, VGPR budget, and in
+  // fp32, whose kernel is kernel 0 with tile_rows set), VALU 32
+  const bool f32 = dtype == BE_F32 && !(flags & BE_PLAN_FORCE_VALU);
+  int rows_cap = mfma ? (d == 256 ? 64 : kMaxTileRows) : f32 ? 64 : kMaxRows;
   if (caps) {
     BE_REQUIRE(!(flags & BE_PLAN_FUSED_MERGE), "the fused merge is not available with a fixed-capacity layout");
     const int tr = caps->tile_rows;
@@ -343,7 +345,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
     BE_REQUIRE(caps->max_items >= 0 && caps->max_queries >= num_queries && caps->max_pages >= 0 &&
                    caps->max_merge >= 0 && caps->max_merge_rows >= 0 && caps->max_zero >= 0,
                "bad plan capacities (max_queries %d < %d queries?)", caps->max_queries, num_queries);
-    if (mfma) rows_cap = std::min(rows_cap, tr);
+    if (mfma || f32) rows_cap = std::min(rows_cap, tr);
   }
   // merge-free row blocks (decode plans, compact layout): forced by
   // BE_PLAN_ROWS, else chosen when rows_preferred says so
@@ -580,7 +582,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   info->dtype = dtype;
   info->kernel = blocks ? 2 : mfma ? 1 : 0;
   info->stream_loop = blocks ? kLoopBlocks : 0;
-  info->tile_rows = blocks ? 128 : caps ? caps->tile_rows : (max_r <= 16 ? 16 : max_r <= 32 ? 32 : max_r <= 64 ? 64 : 128);
+  info->tile_rows = !mfma && !f32 ? 0 : blocks ? 128 : caps ? (f32 ? rows_cap : caps->tile_rows) : (max_r <= 16 ? 16 : max_r <= 32 ? 32 : max_r <= 64 ? 64 : 128);
   info->chunk_tokens = (int32_t)std::min<int64_t>(chunk, INT32_MAX);
   info->plan_ints = (int32_t)off;
   info->off_items = (int32_t)off_items;
@@ -616,6 +618,8 @@ static int launch_attn(const be_attn_plan_info* info, AttnArgs& a, hipStream_t s
     if (info->dtype == BE_F32) return fail(BE_ERR_UNSUPPORTED, "MFMA kernel needs fp16/bf16 storage");
     if (info->tile_rows == kMaxTileRows && block_eligible(info->dtype, info->head_dim)) return block_launch(info, a, st);
     return tile_launch(info, a, st);
+  } else if (info->dtype == BE_F32 && info->tile_rows != 0) {
+    return f32_launch(info, a, st);
   } else {
     switch (info->head_dim) {
       case 64: attn_valu_kernel<T, 64><<<grid, 256, 0, st>>>(a); break;

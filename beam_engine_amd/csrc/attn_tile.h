@@ -237,6 +237,10 @@ inline bool paged4(int page_size, int row_bytes) { return page_size % (1024 / ro
 // hold up to 64 rows: one workgroup per (item, KV head).
 int tile_launch(const be_attn_plan_info* info, const AttnArgs& a, hipStream_t st);
 
+// Launches the fp32 kernel (attn_f32.hip) over a work list whose items hold up to
+// 64 rows: one workgroup per (item, KV head).
+int f32_launch(const be_attn_plan_info* info, const AttnArgs& a, hipStream_t st);
+
 // ---------------------------------------------------------------- 128-row blocks (attn_block.hip)
 // A streaming plan's stream_loop when its causal groups run as 128-row blocks.
 constexpr int kLoopBlocks = 2;

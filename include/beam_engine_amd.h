@@ -200,7 +200,7 @@ typedef struct be_attn_plan_info {
   int32_t num_merge;       /* queries merged by the merge kernel               */
   int32_t num_queries;
   int32_t num_qo_heads, num_kv_heads, head_dim, page_size, num_pages, dtype;
-  int32_t kernel;          /* 0 = VALU, 1 = MFMA tile, 2 = MFMA streaming (persistent),
+  int32_t kernel;          /* 0 = fp32 (MFMA; tile_rows 0: VALU), 1 = MFMA tile, 2 = MFMA streaming (persistent),
                               3 = MFMA row blocks (one kernel, no merge)           */
   int32_t tile_rows;       /* rows (queries x GQA group) per MFMA tile: 16/32  */
   int32_t chunk_tokens;    /* split-K chunk length                             */

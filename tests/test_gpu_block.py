@@ -103,3 +103,15 @@ def test_streaming_plan_when_the_workspace_is_too_small():
     assert full._info.stream_loop == 2 and full._info.partial_bytes > 0
     small = plan(full._need(full._info) - 4096)
     assert small.stats.kernel == "stream" and small._info.stream_loop != 2
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("page", [1, 2, 3, 8, 16])
+@pytest.mark.parametrize("rows", [(4, 1), (20, 2), (3, 32)])
+def test_fp32(ws, d, page, rows):
+    """fp32 storage on the fp32 MFMA kernel: one to four row tiles, all page
+    shapes, within 1e-5 of the float64 oracle."""
+    n, g = rows
+    print(f"[case] f32 rows {n} x {g} d {d} page {page}", flush=True)
+    w = _run(ws, torch.float32, [n, n, 1], [64, 131, 390], 2 * g, 2, d, page)
+    assert w.stats.kernel == "valu" and w._info.tile_rows in (16, 32, 64)
