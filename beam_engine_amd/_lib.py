@@ -206,6 +206,12 @@ def stream_ptr(device=None) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def raw_stream(t: torch.Tensor) -> int:
+    """The current stream of a device tensor's device, as ``stream_ptr`` gives it
+    (without building a Stream object: 0.1 instead of 1.9 us)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
 def require_device(t: torch.Tensor, name: str) -> None:
     if not t.is_cuda:
         raise ValueError(f"{name} must be a HIP device tensor (got {t.device}); there is no CPU path")
