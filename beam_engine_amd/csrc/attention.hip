@@ -192,16 +192,16 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     float m = M;
 #pragma unroll
     for (int u = 0; u < kMergeBatch; ++u) m = fmaxf(m, l[u]);
-    if (m == -INFINITY) continue;                 // nothing seen yet
-    const float s = expf(M - m);
+    const float msafe = m == -INFINITY ? 0.f : m;
+    const float s = expf(M - msafe);              // 0 while nothing was seen
     z *= s;
     acc *= s;
 #pragma unroll
     for (int u = 0; u < kMergeBatch; ++u) {
-      const float wgt = expf(l[u] - m);
+      const float wgt = expf(l[u] - msafe);
       z += wgt;
-      // (a row past the end or one that saw no key holds no finite o to add)
-      if (l[u] != -INFINITY) acc += o[u] * wgt;
+      // a row of NaN scores has lse -inf and o NaN: its o counts, with weight 0
+      if (r0 + u < e) acc += o[u] * wgt;
     }
     M = m;
   }

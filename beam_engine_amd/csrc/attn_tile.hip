@@ -270,6 +270,7 @@ static int launch(const be_attn_plan_info* info, const AttnArgs& a, hipStream_t 
     case 16: BE_TILE_LAUNCH(1) break;
     case 32: BE_TILE_LAUNCH(2) break;
     case 64: BE_TILE_LAUNCH(4) break;
+    case 128: return fail(BE_ERR_UNSUPPORTED, "128-row tiles at head_dim %d", D);
     default: return fail(BE_ERR_INVALID, "corrupt plan: tile_rows %d at head_dim %d", info->tile_rows, D);
   }
 #undef BE_TILE_LAUNCH
