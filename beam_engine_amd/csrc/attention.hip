@@ -414,8 +414,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   // the merge pass (about 8 us) and the fp32 partials' round trip.  The longest
   // query tile is cut into the number of chunks, a power of two, that makes the
   // slower of its own chain and the CUs' shares shortest, those costs included
-  // (1000 fresh tokens, 32 / 8 heads: 32.0 us per layer in two chunks, 28.1
-  // whole).
+  // (1000 fresh tokens, 32 / 8 heads: two chunks take 14% longer than whole).
   int64_t causal_chunk = 0;
   if (any_causal && mfma && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
     int64_t longest = 0, total = 0, queries = 0;

@@ -23,10 +23,10 @@
 // they overlap in part: 2.1 us per tile for a CU's two workgroups, 38% MFMA and
 // 50% VALU busy; a workgroup's prologue and epilogue (about 6 us beside another
 // workgroup's tiles) weigh on short prompts.  Measured on MI355X, us per layer,
-// 32 / 8 heads, head_dim 128: 8 x 1024 tokens 256 (268 TFLOP/s, the streaming
-// kernel's 64-row tiles) -> 101 (681), 4 x 2048 439 -> 167 (823); page 8 fp16,
-// 1500 + 700 + 400 tokens after 400 + 100 + 300 cached 233 (the 16-row-tile
-// kernel, V transposed by 2-byte LDS stores) -> 57.
+// 32 / 8 heads, head_dim 128: 8 x 1024 tokens 252 (272 TFLOP/s, the streaming
+// kernel's 64-row tiles) -> 103 (666), 4 x 2048 439 -> 179 (769); page 8 fp16,
+// three ragged prompts of up to 1500 tokens after up to 400 cached 292 (the
+// 16-row-tile kernel, V transposed by 2-byte LDS stores) -> 66.
 
 #include <math.h>
 
@@ -80,11 +80,6 @@ __device__ __forceinline__ float other_half_sum(float x) {
   const unsigned a = r.x, b = r.y;
   return __uint_as_float(a) + __uint_as_float(b);
 }
-
-// A row's running max may lag the true one by this much (log2 units) before its
-// sums are rescaled: P and l grow by at most 2^8, far inside the range of the
-// 16-bit P and the fp32 sums, with the same relative rounding.
-constexpr float kLag = 8.f;
 
 template <typename T, int D, bool PAGED4>
 __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_items) {
@@ -229,7 +224,10 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
       for (int i = 0; i < 16; i += 2)
         mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[tb][i], x[tb][i + 1]), mx);
     mx = other_half_max(mx) * scale;
-    if (__builtin_amdgcn_ballot_w64(mx > m_run + kLag) != 0) {
+    // (the running max follows the true one at once, so that a row's largest
+    // weight is exactly 1: letting it lag by up to 2^8 saved 4%, 99.8 -> 96.1 us at 8
+    // x 1024 tokens, but was 3% further from the 64-bit result in fp16)
+    if (__builtin_amdgcn_ballot_w64(mx > m_run) != 0) {
       const float m_new = fmaxf(m_run, mx);
       const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
       l_run *= alpha;

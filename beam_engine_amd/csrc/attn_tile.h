@@ -247,9 +247,9 @@ constexpr int kLoopBlocks = 2;
 // Blocks (query tiles x KV heads) of a causal plan from which it does: below,
 // the streaming kernel's split of the keys over all CUs is as fast or faster.  One
 // bf16 prompt at 32 / 8 heads, head_dim 128, MI355X, streaming -> blocks: 256
-// tokens (64 blocks) 13.8 -> 11.3 us, 512 23.1 -> 16.0, 1000 46.7 -> 28.1, 3000
-// 243.6 -> 87 - 93; 8 x 1024 tokens 256 -> 101; 8 / 8 heads, 1000 tokens (64
-// blocks) 21.5 -> 21.6.
+// tokens (64 blocks) 13.8 -> 11.0 us, 512 23.1 -> 17.4, 1000 46.7 -> 30.4, 3000
+// 243.6 -> 112; 8 x 1024 tokens 252 -> 103; 8 / 8 heads, 1000 tokens (64 blocks)
+// about even.
 constexpr int64_t kMinCausalBlocks = 64;
 
 // True when the block kernel has an instantiation for this shape.
