@@ -93,7 +93,7 @@ class BeTreeModel(ctypes.Structure):
 
 
 EXPORTS = (
-    "be_version", "be_last_error", "be_kv_append", "be_rope_qkv_append", "be_page_copy", "be_page_copy_counted",
+    "be_version", "be_last_error", "be_kv_append", "be_rope_qkv_append", "be_add_rms_norm", "be_silu_mul", "be_page_copy", "be_page_copy_counted",
     "be_attn_plan",
     "be_attn_run",
     "be_merge_states", "be_beam_topk_workspace_bytes", "be_beam_topk", "be_beam_topk_noalloc", "be_trie_cascade",
@@ -127,6 +127,8 @@ def load() -> ctypes.CDLL:
     lib.be_kv_append.argtypes = [vp, i32, i32, i32, i32, i32, vp, vp, vp, i64, i64, vp, i64, i64, i32, vp, vp]
     lib.be_rope_qkv_append.argtypes = [vp, i64, i32, i32, i32, i32, i32, vp, vp, vp, i32, vp, vp, i32, i32, vp, vp,
                                        vp, vp]
+    lib.be_add_rms_norm.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, ctypes.c_float, vp]
+    lib.be_silu_mul.argtypes = [vp, vp, i32, i32, i32, vp]
     lib.be_page_copy.argtypes = [vp, i64, i32, i32, i32, i32, i32, i32, vp, vp, vp, i32, vp, vp]
     lib.be_page_copy_counted.argtypes = [vp, i64, i32, i32, i32, i32, i32, i32, vp, vp, vp, vp, i32, vp, vp]
     lib.be_attn_plan.argtypes = [ctypes.POINTER(BeLevel), i32, i32, i32, i32, i32, i32, i32, i32, i32, i32,

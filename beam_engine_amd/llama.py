@@ -27,6 +27,8 @@ from typing import Callable, List, Optional
 import torch
 import torch.nn.functional as F
 
+from . import _lib
+
 
 @dataclass
 class LlamaConfig:
@@ -96,6 +98,27 @@ class LlamaDecoder:
     def _rms(self, x: torch.Tensor, wgt: torch.Tensor) -> torch.Tensor:
         return F.rms_norm(x, (x.shape[-1],), wgt, self.cfg.rms_norm_eps)
 
+    def _add_rms(self, x: torch.Tensor, delta: Optional[torch.Tensor], wgt: torch.Tensor):
+        """(x + delta, its RMSNorm); without ``delta`` (x, its RMSNorm).  16-bit
+        storage: one kernel, with the tensor code's roundings."""
+        if delta is None:
+            return x, self._rms(x, wgt)
+        n = x.shape[-1]
+        if not (self._fusable(x, delta, wgt) and x.shape == delta.shape and n <= 8192):
+            x = x + delta
+            return x, self._rms(x, wgt)
+        s, h = torch.empty_like(x), torch.empty_like(x)
+        _lib.check(_lib.load().be_add_rms_norm(x.data_ptr(), delta.data_ptr(), wgt.data_ptr(), s.data_ptr(), h.data_ptr(),
+                                               _lib.dtype_code(x.dtype), x.numel() // n, n, self.cfg.rms_norm_eps,
+                                               _lib.raw_stream(x)), "add_rms_norm")
+        return s, h
+
+    @staticmethod
+    def _fusable(*ts: torch.Tensor) -> bool:
+        dt = ts[0].dtype
+        return dt in (torch.float16, torch.bfloat16) and ts[0].shape[-1] % 8 == 0 and ts[0].numel() > 0 and \
+            all(t.is_cuda and t.dtype == dt and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in ts)
+
     @staticmethod
     def _rotate_half(x):
         x1, x2 = x.chunk(2, dim=-1)
@@ -116,11 +139,18 @@ class LlamaDecoder:
         v = qkv[..., (hq + hkv) * d:].unflatten(-1, (hkv, d))
         return q, k, v
 
-    def _mlp(self, layer, x):
-        h = self._rms(x, layer["ln2"])
+    def _mlp(self, layer, h):
+        """The gated MLP of normalised rows (before the residual add)."""
         gu = F.linear(h, layer["wgu"])
-        g, u = gu.chunk(2, dim=-1)
-        return x + F.linear(F.silu(g) * u, layer["wd"])
+        n = gu.shape[-1] // 2
+        if self._fusable(gu) and n % 8 == 0:
+            y = torch.empty((*gu.shape[:-1], n), dtype=gu.dtype, device=gu.device)
+            _lib.check(_lib.load().be_silu_mul(gu.data_ptr(), y.data_ptr(), _lib.dtype_code(gu.dtype), y.numel() // n, n,
+                                               _lib.raw_stream(gu)), "silu_mul")
+        else:
+            g, u = gu.chunk(2, dim=-1)
+            y = F.silu(g) * u
+        return F.linear(y, layer["wd"])
 
     # ---------------------------------------------------------------- prefill
     @torch.no_grad()
@@ -146,9 +176,9 @@ class LlamaDecoder:
         pre.plan([i * s for i in range(r + 1)], [i * npg for i in range(r + 1)],
                  [p[j] for p in page_ids for j in range(npg)], [s - (npg - 1) * ps] * r, hq, hkv, d, ps,
                  causal=True, q_data_type=self.dtype)
-        x = F.embedding(input_ids, self.embed)
+        x, y = F.embedding(input_ids, self.embed), None
         for li, layer in enumerate(self.layers):
-            h = self._rms(x, layer["ln1"])
+            x, h = self._add_rms(x, y, layer["ln1"])
             if fused:
                 # RoPE and the append as one pass over the projections, bit-identical
                 # to the tensor code below (its table gathers, products, concatenations
@@ -162,9 +192,9 @@ class LlamaDecoder:
                 page_table.write_blocks_vectorized(li, pages, k.reshape(r * s, hkv, d).contiguous(),
                                                    v.reshape(r * s, hkv, d).contiguous(), slots)
             o = pre.run(q.reshape(r * s, hq, d), page_table.kv_cache_at_layer[li]).reshape(r, s, hq * d)
-            x = x + F.linear(o, layer["wo"])
-            x = self._mlp(layer, x)
-        last = self._rms(x[:, -1], self.norm)
+            x, h = self._add_rms(x, F.linear(o, layer["wo"]), layer["ln2"])
+            y = self._mlp(layer, h)
+        last = self._rms(x[:, -1] if y is None else x[:, -1] + y[:, -1], self.norm)
         return F.linear(last, self.lm_head)
 
     # ---------------------------------------------------------------- decode
@@ -178,9 +208,9 @@ class LlamaDecoder:
         logits [N, V]."""
         n = token_ids.shape[0]
         cfg = self.cfg
-        x = F.embedding(token_ids, self.embed)
+        x, y = F.embedding(token_ids, self.embed), None
         for li, layer in enumerate(self.layers):
-            h = self._rms(x, layer["ln1"])
+            x, h = self._add_rms(x, y, layer["ln1"])
             if fused_rope:
                 qkv = F.linear(h, layer["wqkv"])
                 q = page_table.write_rope_qkv(li, qkv, cfg.num_attention_heads, positions, self.cos, self.sin,
@@ -191,9 +221,9 @@ class LlamaDecoder:
                 k = self._rope(k, positions)
                 page_table.write_blocks_vectorized(li, write_pages, k, v, write_pos)
             o = attn(li, q, page_table.kv_cache_at_layer[li])
-            x = x + F.linear(o.reshape(n, -1), layer["wo"])
-            x = self._mlp(layer, x)
-        return F.linear(self._rms(x, self.norm), self.lm_head)
+            x, h = self._add_rms(x, F.linear(o.reshape(n, -1), layer["wo"]), layer["ln2"])
+            y = self._mlp(layer, h)
+        return F.linear(self._add_rms(x, y, self.norm)[1], self.lm_head)
 
 
 def _align(nbytes: int, to: int = 256) -> int:
@@ -271,15 +301,16 @@ class GraphedDecoder:
     def _segment(self, l: int, x: Optional[torch.Tensor]):
         m, cfg = self.model, self.model.cfg
         if l == 0:
-            x = F.embedding(self.tok, m.embed)
+            x, y = F.embedding(self.tok, m.embed), None
         else:
             prev = m.layers[l - 1]
-            x = x + F.linear(self.o.reshape(self.n, -1), prev["wo"])
-            x = m._mlp(prev, x)
+            x, h = m._add_rms(x, F.linear(self.o.reshape(self.n, -1), prev["wo"]), prev["ln2"])
+            y = m._mlp(prev, h)
         if l == cfg.num_hidden_layers:
-            return x, None, F.linear(m._rms(x, m.norm), m.lm_head)
+            x, h = m._add_rms(x, y, m.norm)
+            return x, None, F.linear(h, m.lm_head)
         layer = m.layers[l]
-        h = m._rms(x, layer["ln1"])
+        x, h = m._add_rms(x, y, layer["ln1"])
         qkv = F.linear(h, layer["wqkv"])
         q = self.pt.write_rope_qkv(l, qkv, cfg.num_attention_heads, self.pos, m.cos, m.sin, self.wpg, self.wps)
         return x, q, None

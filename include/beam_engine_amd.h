@@ -129,6 +129,17 @@ int be_rope_qkv_append(const void* qkv, int64_t qkv_stride_n, int dtype, int n, 
                        void* kv_layer, int num_pages, int page_size, const int32_t* page_idx,
                        const int32_t* slot, int32_t* err_count, void* stream);
 
+/* be_add_rms_norm: the decoder's residual add and the RMSNorm that reads it, one
+ * pass over contiguous [rows, n] 16-bit tensors: sum = round(x + delta), out =
+ * round(sum * rsqrt(mean(sum^2) + eps) * weight[n]) in fp32.  n: a multiple of 8
+ * up to 8192; operands 16-byte aligned; sum and out may be x or delta. */
+int be_add_rms_norm(const void* x, const void* delta, const void* weight, void* sum, void* out, int dtype,
+                    int rows, int n, float eps, void* stream);
+
+/* be_silu_mul: out [rows, n] = round(round(SiLU(gate)) * up) of contiguous 16-bit
+ * rows [gate (n) | up (n)].  n: a multiple of 8; operands 16-byte aligned. */
+int be_silu_mul(const void* gate_up, void* out, int dtype, int rows, int n, void* stream);
+
 /* ------------------------------------------------------------------ attention
  * One level of a cascade (FlashInfer's per-level index arrays as built by
  * BeamState.get_cascade_input, src/beam_engine/beam_state.py:211-412): group
