@@ -6,7 +6,8 @@
 // was two kernels and the second read back what the first had just written.
 // MI355X, 2 x 512 prompt tokens, bf16: SiLU and product over 1024 x 14336 22.4 + 18.1
 // -> 19.4 us (4.5 TB/s), add and norm over 1024 x 4096 5.8 + 8.9 -> 8.7 us (3.9
-// TB/s); that prefill call 1392 -> 1345 us over two layers.
+// TB/s); that prefill call 1392 -> 1345 us over two layers; a decode step of 128
+// candidates through 32 layers 7.11 -> 6.62 ms.
 // Roundings are the tensor code's: the sum to the storage type before the norm
 // reads it, SiLU to the storage type before the product.
 
