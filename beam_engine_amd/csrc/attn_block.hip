@@ -23,12 +23,14 @@
 // they overlap in part: 2.1 us per tile for a CU's two workgroups, 38% MFMA and
 // 50% VALU busy; a workgroup's prologue and epilogue (about 6 us beside another
 // workgroup's tiles) weigh on short prompts.  Measured on MI355X, us per layer,
-// 32 / 8 heads, head_dim 128: 8 x 1024 tokens 252 (272 TFLOP/s, the streaming
-// kernel's 64-row tiles) -> 103 (666), 4 x 2048 439 -> 179 (769); page 8 fp16,
-// three ragged prompts of up to 1500 tokens after up to 400 cached 292 (the
-// 16-row-tile kernel, V transposed by 2-byte LDS stores) -> 66.
+// 32 / 8 heads, head_dim 128: 8 x 1024 tokens 250 (275 TFLOP/s, the streaming
+// kernel's 64-row tiles) -> 92 to 99 (695 to 748), 4 x 2048 436 -> 157 to 167 (823
+// to 876); page 8 fp16, three ragged prompts of up to 1500 tokens after up to 400
+// cached 292 (the 16-row-tile kernel, V transposed by 2-byte LDS stores) -> 64.
 
 #include <math.h>
+
+#include <type_traits>
 
 #include "attn_tile.h"
 
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
       voff[mb][u] = vr * RB + (((mb * 4 + e4) ^ swz<D>(vr)) << 4) + (r16 & 1) * 8;
     }
 
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, m_top = -INFINITY, l_run = 0.f;   // reference of the sums, the largest score, the weights' sum
   v16f o_acc[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
@@ -170,14 +172,15 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
     for (int i = 0; i < 16; ++i) o_acc[mb][i] = 0.f;
 
   const int n_tiles = (it.tok_count + kTile - 1) / kTile;
-  for (int tile = 0; tile < n_tiles; ++tile) {
+  auto step = [&](auto one, int tile) {
+    constexpr bool ONE = decltype(one)::value;       // the item's only tile
     const int st = tile & 1;
     // this wave's loads of the tile have landed; after the barrier everyone's
     // have, and everyone is done with the other stage
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (tile + 1 < n_tiles) ld.load(lds0 + (st ^ 1) * STAGE);
+    if (!ONE && tile + 1 < n_tiles) ld.load(lds0 + (st ^ 1) * STAGE);
     const int t0 = tile * kTile;
-    if (!wave_on || t0 >= lim_most) continue;
+    if (!wave_on || t0 >= lim_most) return;
     const unsigned char* kt = stage + st * STAGE;
     const unsigned char* vt = kt + PLANE;
 
@@ -217,44 +220,66 @@ __global__ __launch_bounds__(256, 2) void attn_block_kernel(AttnArgs a, int n_it
     }
     // (maximum rather than fmax: no canonicalising of the MFMA results; a NaN
     // score makes the row NaN either way)
-    float mx = -INFINITY;
+    float mx[2] = {-INFINITY, -INFINITY};
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
       for (int i = 0; i < 16; i += 2)
-        mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[tb][i], x[tb][i + 1]), mx);
-    mx = other_half_max(mx) * scale;
-    // (the running max follows the true one at once, so that a row's largest
-    // weight is exactly 1: letting it lag by up to 2^8 saved 4%, 99.8 -> 96.1 us at 8
-    // x 1024 tokens, but was 3% further from the 64-bit result in fp16)
-    if (__builtin_amdgcn_ballot_w64(mx > m_run) != 0) {
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
-      l_run *= alpha;
+        mx[tb] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(x[tb][i], x[tb][i + 1]), mx[tb]);
+    // When a row's largest score (m_top) grows, every row of the wave takes the
+    // tile's largest as its reference -- in an item's only tile each 32-token
+    // block's -- so that this weight is exactly 1 in the 16-bit P, unless it lies
+    // 2^8 below m_top: weights, l and Oᵀ stay within 2^8 of their scale at m_top.
+    // With m_top itself as the reference only the row's largest weight is exact,
+    // where the streaming kernel, which splits the tokens over two waves, has two:
+    // bf16 prompts were 2.00e-3 from the 64-bit result against 1.98e-3 (8 x 1024
+    // tokens; 1.96e-3 now) and 1.84e-3 against 1.83e-3 (8 x 64; 1.83e-3 now).  It
+    // costs 0 to 2% of the launch (8 x 1024 tokens 91.4 -> 91.7 us, 512 35.9 -> 36.6).
+    auto refer = [&](float top) {
+      top = other_half_max(top) * scale;
+      if (__builtin_amdgcn_ballot_w64(top > m_top) != 0) {
+        m_top = fmaxf(m_top, top);
+        const float m_new = top >= m_top - 8.f ? top : m_run;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - (m_new == -INFINITY ? 0.f : m_new));
+        l_run *= alpha;
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) o_acc[mb] *= alpha;
-      m_run = m_new;
-    }
-    const float msafe = m_run == -INFINITY ? 0.f : m_run;
-    v8s pf[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      uint32_t pw[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(x[s >> 1][8 * (s & 1) + 2 * j], scale, -msafe));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(x[s >> 1][8 * (s & 1) + 2 * j + 1], scale, -msafe));
-        l_run += p0 + p1;
-        pw[j] = pack2<T>(p0, p1);
+        for (int mb = 0; mb < MB; ++mb) o_acc[mb] *= alpha;
+        m_run = m_new;
       }
-      typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-      pf[s] = __builtin_bit_cast(v8s, (u4){pw[0], pw[1], pw[2], pw[3]});
+    };
+    constexpr int NB = ONE ? 1 : 2;                  // 32-token blocks per reference
+#pragma unroll
+    for (int b = 0; b < 2; b += NB) {
+      refer(ONE ? mx[b] : __builtin_elementwise_maximum(mx[0], mx[1]));
+      const float msafe = m_run == -INFINITY ? 0.f : m_run;
+      v8s pf[2 * NB];
+#pragma unroll
+      for (int s = 0; s < 2 * NB; ++s) {
+        const int tb = b + (s >> 1);
+        uint32_t pw[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float p0 = __builtin_amdgcn_exp2f(fmaf(x[tb][8 * (s & 1) + 2 * j], scale, -msafe));
+          const float p1 = __builtin_amdgcn_exp2f(fmaf(x[tb][8 * (s & 1) + 2 * j + 1], scale, -msafe));
+          l_run += p0 + p1;
+          pw[j] = pack2<T>(p0, p1);
+        }
+        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+        pf[s] = __builtin_bit_cast(v8s, (u4){pw[0], pw[1], pw[2], pw[3]});
+      }
+#pragma unroll
+      for (int s = 0; s < 2 * NB; ++s)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const v4s *v = vf[2 * b + s][mb];
+          o_acc[mb] = mfma32<T>(__builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7), pf[s], o_acc[mb]);
+        }
     }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        o_acc[mb] = mfma32<T>(__builtin_shufflevector(vf[s][mb][0], vf[s][mb][1], 0, 1, 2, 3, 4, 5, 6, 7), pf[s], o_acc[mb]);
+  };
+  if (n_tiles == 1) {
+    step(std::true_type(), 0);
+  } else {
+    for (int tile = 0; tile < n_tiles; ++tile) step(std::false_type(), tile);
   }
 
   // ---- writes: lane holds Oᵀ[32 mb + 8 (i / 4) + 4 h + i % 4][row]
