@@ -182,8 +182,8 @@ class _PagedPlanner:
             # (a capacity error with plan_ints 0 is a fixed layout's, which no
             # buffer size cures: MemoryError)
             _lib.check(rc, "attention plan")
-            if info.kernel == 2 and info.stream_loop == 2 and self._need(info) > self._ws.numel():
-                flags |= _lib.BE_PLAN_NO_BLOCKS       # the streaming plan's 16-bit slots may still fit
+            if self._less_scratch(info, flags):
+                flags |= _lib.BE_PLAN_LESS_SCRATCH
                 continue
             break
         self._install_plan(info, buf, staging, max_page, head_dim, sm_scale, q_data_type)
@@ -192,6 +192,11 @@ class _PagedPlanner:
     def _need(info) -> int:
         """Workspace bytes of a plan: its words, then the partial rows."""
         return (int(info.plan_ints) * 4 + _WS_ALIGN - 1) // _WS_ALIGN * _WS_ALIGN + int(info.partial_bytes)
+
+    def _less_scratch(self, info, flags: int) -> bool:
+        """Whether to plan again with BE_PLAN_LESS_SCRATCH: the plan does not fit
+        the workspace and was made without it."""
+        return self._need(info) > self._ws.numel() and not flags & _lib.BE_PLAN_LESS_SCRATCH
 
     def _plan_flags(self) -> int:
         return (_lib.BE_PLAN_FORCE_VALU if self._force_valu else 0) | \

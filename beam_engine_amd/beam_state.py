@@ -937,13 +937,14 @@ class NativeBeamState:
         pm = ctypes.byref(model) if model is not None else None
         code = _lib.KIND_CODES[kind]
         cap = host_plan.numel() if host_plan is not None else staging.buf.numel()
+        flags = wrapper._plan_flags()
         while True:
             buf = host_plan if host_plan is not None else staging.acquire(cap)
             meta = self._meta_buf
             if self._meta_ptr[0] is not meta:
                 self._meta_ptr = (meta, meta.ctypes.data)
             rc = self._lib.be_trie_plan_kind(self._h, code, int(include_self), pm, num_qo_heads, num_kv_heads,
-                                             head_dim, _lib.dtype_code(q_data_type), wrapper._plan_flags(),
+                                             head_dim, _lib.dtype_code(q_data_type), flags,
                                              wrapper._num_cus or _num_cus(wrapper._ws.device), caps,
                                              self._meta_ptr[1], meta.size, ctypes.byref(self._meta_used),
                                              buf.data_ptr(), buf.numel(), ctypes.byref(info), ctypes.byref(max_page),
@@ -959,6 +960,9 @@ class NativeBeamState:
                     _lib.check(rc, f"{kind} plan")
                 continue
             _lib.check(rc, f"{kind} plan")
+            if wrapper._less_scratch(info, flags):
+                flags |= _lib.BE_PLAN_LESS_SCRATCH
+                continue
             break
         wrapper.num_levels = int(self._meta_buf[0])
         wrapper._install_plan(info, buf, staging, int(max_page.value), head_dim, None, q_data_type,

@@ -336,7 +336,11 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   // rows per workgroup: MFMA 8 row tiles (4 at head_dim 256, VGPR budget, and in
   // fp32, whose kernel is kernel 0 with tile_rows set), VALU 32
   const bool f32 = dtype == BE_F32 && !(flags & BE_PLAN_FORCE_VALU);
-  int rows_cap = mfma ? (d == 256 ? 64 : kMaxTileRows) : f32 ? 64 : kMaxRows;
+  // (fp32 on 64-row items: half the K / V reads, but half the items too, so more
+  // key splits and fp32 partial rows; a 1000-token prompt, 32 / 8 heads, head_dim
+  // 128, takes 9.8 MB of workspace where 32-row items take 12.5 KB)
+  const bool less = (flags & BE_PLAN_LESS_SCRATCH) != 0;
+  int rows_cap = mfma ? (d == 256 ? 64 : kMaxTileRows) : f32 && !less ? 64 : kMaxRows;
   if (caps) {
     BE_REQUIRE(!(flags & BE_PLAN_FUSED_MERGE), "the fused merge is not available with a fixed-capacity layout");
     const int tr = caps->tile_rows;
@@ -376,7 +380,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   for (const Group& gr : groups)
     if (gr.kv_len > 0 && is_causal(gr)) causal_blocks += ceil_div(gr.q1 - gr.q0, q_tile) * hkv;
   const bool streams = stream_eligible(dtype, d, g, page_size, flags);
-  const bool blocks = streams && !caps && !(flags & BE_PLAN_NO_BLOCKS) && causal_blocks >= kMinCausalBlocks;
+  const bool blocks = streams && !caps && !less && !(flags & BE_PLAN_NO_BLOCKS) && causal_blocks >= kMinCausalBlocks;
   if (!(any_causal && caps) && streams && !blocks && (!caps || caps->tile_rows == 64)) {
     memset(info, 0, sizeof(*info));
     const int rc = stream_plan(groups, levels, num_levels, total_pages, num_queries, hq, hkv, d, page_size,
@@ -416,7 +420,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   // slower of its own chain and the CUs' shares shortest, those costs included
   // (1000 fresh tokens, 32 / 8 heads: two chunks take 14% longer than whole).
   int64_t causal_chunk = 0;
-  if (any_causal && mfma && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
+  if (any_causal && mfma && !less && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
     int64_t longest = 0, total = 0, queries = 0;
     for (const Group& gr : groups) {
       if (gr.kv_len <= 0 || gr.q1 <= gr.q0) continue;

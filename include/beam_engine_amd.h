@@ -191,6 +191,10 @@ typedef struct be_level {
 #define BE_PLAN_NO_BLOCKS 4096   /* causal groups stay on the streaming kernel where it applies
                                     (by default plans with many query rows run as 128-row
                                     blocks, whose split keys take fp32 partial rows)         */
+#define BE_PLAN_LESS_SCRATCH 8192 /* for a workspace that the default plan does not fit: causal
+                                    groups on the streaming kernel where it applies (16-bit
+                                    partials) and elsewhere cut as decode groups are, fp32
+                                    groups in 32-row tiles (half as many key splits)         */
 
 /* Fixed-capacity plan layout (for HIP-graph capture): every region of the
  * device plan sits at an offset that depends only on these capacities, the

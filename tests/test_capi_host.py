@@ -642,6 +642,22 @@ def test_causal_block_plan_covers_visible_tokens(q_lens, cached, hq, hkv, cus):
     assert rc == 0 and (info.kernel, info.stream_loop) != (2, 2)
 
 
+@pytest.mark.parametrize("d,page,tokens,dtype,fits", [(128, 16, 1000, 0, 12_544), (128, 32, 1000, 0, 12_288)])
+def test_less_scratch_fp32_plan(d, page, tokens, dtype, fits):
+    """fp32 prompts on 64-row items are cut into more key splits than on 32-row
+    items; BE_PLAN_LESS_SCRATCH plans the latter, whose workspace (``fits``: plan
+    words and partial rows, bytes) needs no partial rows here."""
+    npg = -(-tokens // page)
+    levels = [([0, tokens], [0, npg], list(range(npg)), [tokens - (npg - 1) * page])]
+
+    def need(flags):
+        rc, info, _, _, L = plan(levels, hq=32, hkv=8, d=d, page=page, num_pages=npg, dtype=dtype, flags=128 | flags)
+        assert rc == 0, L.be_last_error()
+        assert info.kernel == 0 and info.tile_rows in (16, 32, 64)
+        return -(-info.plan_ints * 4 // 256) * 256 + info.partial_bytes
+    assert need(8192) <= fits < need(0)
+
+
 # ---------------------------------------------------------------- row-block plans
 ROWS = 256     # BE_PLAN_ROWS
 

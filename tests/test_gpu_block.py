@@ -89,20 +89,36 @@ def test_keys_split_over_blocks(ws, page):
     assert w.stats.num_merge == 40
 
 
-def test_streaming_plan_when_the_workspace_is_too_small():
+@pytest.mark.parametrize("dtype,hq,hkv,page,n,kv_len,small", [
+    (torch.bfloat16, 32, 8, 16, 256, 8256, "stream"), (torch.float32, 32, 8, 16, 1000, 1000, "f32")])
+def test_plan_for_a_small_workspace(dtype, hq, hkv, page, n, kv_len, small):
     """A causal plan whose fp32 partial rows do not fit the workspace is planned
-    for the streaming kernel, whose 16-bit slots do."""
+    again with less scratch: 16-bit storage for the streaming kernel, fp32 in
+    32-row items.  Both plans run."""
     from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
-    (qo, kvp, kvi, lpl), pages = _levels([256], [8256], 16)
+    print(f"[case] small workspace {dtype}", flush=True)
+    d = 128
+    (qo, kvp, kvi, lpl), pages = _levels([n], [kv_len], page)
+    g = torch.Generator().manual_seed(4)
+    kv = torch.randn((pages, 2, page, hkv, d), generator=g).to(dtype)
+    q = torch.randn((n, hq, d), generator=g).to(dtype)
+    ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, None, causal=True)
 
-    def plan(nbytes):
+    def run(nbytes):
         w = BatchPrefillWithPagedKVCacheWrapper(torch.empty(nbytes, dtype=torch.uint8, device="cuda"))
-        w.plan(qo, kvp, kvi, lpl, 32, 8, 128, 16, causal=True, q_data_type=torch.bfloat16)
+        w.plan(qo, kvp, kvi, lpl, hq, hkv, d, page, causal=True, q_data_type=dtype)
+        out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
+        torch.cuda.synchronize()
+        _check(out, lse, ref_o, ref_lse, dtype)
         return w
-    full = plan(256 << 20)
-    assert full._info.stream_loop == 2 and full._info.partial_bytes > 0
-    small = plan(full._need(full._info) - 4096)
-    assert small.stats.kernel == "stream" and small._info.stream_loop != 2
+    full = run(256 << 20)
+    assert full._info.partial_bytes > 8 << 20
+    less = run(full._need(full._info) - 4096)
+    assert less._need(less._info) < full._need(full._info)
+    if small == "stream":
+        assert full._info.stream_loop == 2 and less._info.kernel == 2 and less._info.stream_loop != 2
+    else:
+        assert full._info.tile_rows == 64 and less._info.tile_rows == 32
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
