@@ -349,7 +349,10 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
     BE_REQUIRE(caps->max_items >= 0 && caps->max_queries >= num_queries && caps->max_pages >= 0 &&
                    caps->max_merge >= 0 && caps->max_merge_rows >= 0 && caps->max_zero >= 0,
                "bad plan capacities (max_queries %d < %d queries?)", caps->max_queries, num_queries);
-    if (mfma || f32) rows_cap = std::min(rows_cap, tr);
+    if (mfma) rows_cap = std::min(rows_cap, tr);
+    // (fp32: never more items than 32-row ones, which capacities were sized for
+    // whatever tile_rows said; causal ones cut their keys by their own rows)
+    if (f32 && (tr <= 32 || any_causal)) rows_cap = kMaxRows;
   }
   // merge-free row blocks (decode plans, compact layout): forced by
   // BE_PLAN_ROWS, else chosen when rows_preferred says so
@@ -402,9 +405,11 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   }
 
   // ---- split-K chunk: about two workgroups per CU over all (tile, chunk, head)
+  // (fixed fp32 layouts: cut as 32-row items, so that partial rows stay as many)
+  const int cut_tile = caps && f32 ? std::max(1, kMaxRows / g) : q_tile;
   int64_t work = 0;   // token-tiles
   for (const Group& gr : groups)
-    if (gr.q1 > gr.q0 && gr.kv_len > 0) work += ceil_div(gr.q1 - gr.q0, q_tile) * (int64_t)gr.kv_len;
+    if (gr.q1 > gr.q0 && gr.kv_len > 0) work += ceil_div(gr.q1 - gr.q0, cut_tile) * (int64_t)gr.kv_len;
   const int64_t target = 3 * (int64_t)num_cus;
   int64_t chunk = ceil_div(work * hkv, target);
   chunk = std::max<int64_t>(128, ceil_div(chunk, 64) * 64);

@@ -203,7 +203,8 @@ typedef struct be_level {
  * fails with BE_ERR_CAPACITY. */
 typedef struct be_plan_caps {
   int32_t max_items, max_queries, max_pages, max_merge, max_merge_rows, max_zero;
-  int32_t tile_rows;       /* fixed rows per workgroup tile: 16, 32, 64 or 128 */
+  int32_t tile_rows;       /* fixed rows per workgroup tile: 16, 32, 64 or 128 (fp32: 32-row
+                              items up to 32 and with a causal group, else 64) */
   int32_t max_tails;       /* streaming kernel: tail chunk entries (and tail-role items) */
 } be_plan_caps;
 

@@ -658,6 +658,27 @@ def test_less_scratch_fp32_plan(d, page, tokens, dtype, fits):
     assert need(8192) <= fits < need(0)
 
 
+@pytest.mark.parametrize("tile_rows", [16, 32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fixed_fp32_layout_takes_no_more_than_32_row_items(tile_rows, causal):
+    """fp32 fixed layouts stay within the capacities that 32-row items need,
+    whatever tile_rows: 64 queries over 500 tokens, 8 / 2 heads, are 8 items of 8
+    queries on 16 of a group, causal prompts (2 x 70 queries) 9 tiles each."""
+    _lib, _ = lib()
+    if causal:
+        levels, nq = [([0, 70, 140], [0, 5, 10], list(range(10)), [6, 6])], 140
+        items = 2 * 9
+    else:
+        levels, nq = [([0, 64], [0, 32], list(range(32)), [4])], 64
+        items = 8 * 4                                  # four 128-token chunks
+    rows = 0 if causal else 64 * 4
+    caps = _lib.BePlanCaps(items, nq, 32, 0 if causal else 64, rows, 0, tile_rows, 0)
+    rc, info, buf, _, L = plan(levels, page=16, num_pages=32, dtype=0, flags=128 if causal else 0, caps=caps)
+    assert rc == 0, L.be_last_error()
+    assert info.num_items <= items and info.tile_rows in (32, 64)
+    assert (decode_items(info, buf)[:, 1] * 4 <= info.tile_rows).all()
+
+
 # ---------------------------------------------------------------- row-block plans
 ROWS = 256     # BE_PLAN_ROWS
 

@@ -161,6 +161,23 @@ def test_fp32(ws, d, page, rows):
     assert w.stats.kernel == "valu" and w._info.tile_rows in (16, 32, 64)
 
 
+@pytest.mark.parametrize("tile_rows", [16, 32, 64])
+def test_fp32_fixed_layout(ws, tile_rows):
+    """fp32 in a fixed-capacity layout sized for 32-row items."""
+    from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
+    print(f"[case] f32 fixed layout {tile_rows}", flush=True)
+    (qo, kvp, kvi, lpl), pages = _levels([64], [500], 16)
+    g = torch.Generator().manual_seed(6)
+    kv = torch.randn((pages, 2, 16, 2, 128), generator=g)
+    q = torch.randn((64, 8, 128), generator=g)
+    w = BatchPrefillWithPagedKVCacheWrapper(ws)
+    w.use_fixed_layout(32, 64, 32, 64, 256, 0, tile_rows)
+    w.plan(qo, kvp, kvi, lpl, 8, 2, 128, 16, causal=False, q_data_type=torch.float32)
+    out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
+    ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], 16, None)
+    _check(out, lse, ref_o, ref_lse, torch.float32)
+
+
 @pytest.mark.parametrize("dtype,d,page,n", [(torch.bfloat16, 64, 8, 4), (torch.float32, 64, 16, 4), (torch.float32, 128, 16, 4),
                                             (torch.bfloat16, 64, 16, 64)])
 @pytest.mark.parametrize("where", ["k", "v"])
