@@ -159,6 +159,9 @@ class LlamaDecoder:
         token's K/V into the request's pages; returns last-position logits [R, V]."""
         cfg = self.cfg
         r, s = input_ids.shape
+        if s > self.cos.shape[0]:
+            # (the RoPE append only counts positions beyond its tables)
+            raise ValueError(f"prompts of {s} tokens, the RoPE tables hold {self.cos.shape[0]} positions")
         hq, hkv, d = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
         ps = page_table.page_size
         pos = torch.arange(s, device=self.device).unsqueeze(0).expand(r, s)
