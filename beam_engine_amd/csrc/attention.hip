@@ -34,9 +34,11 @@ struct MergeArgs {
 };
 
 // ================================================================== VALU kernel
-// Any storage dtype, D in {64, 128, 256}, up to 32 rows per tile.  K/V blocks
-// of 32 tokens are converted to fp32 in LDS; scores use one thread per
-// (token, row-group), P.V one thread per (head_dim column, row-group).
+// Any storage dtype and alignment, D in {64, 128, 256}, up to 32 rows per
+// workgroup (blockIdx.z picks them from items of more).  K/V blocks of 32 tokens
+// are converted to fp32 in LDS; scores use one thread per (token, row-group), P.V
+// one thread per (head_dim column, row-group).  Runs BE_PLAN_FORCE_VALU plans, and
+// any work list whose operands the other kernels' 16-byte accesses cannot take.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void attn_valu_kernel(AttnArgs a) {
   constexpr int BT = 32;
@@ -50,10 +52,16 @@ __global__ __launch_bounds__(256) void attn_valu_kernel(AttnArgs a) {
   __shared__ float alpha_s[kMaxRows], l_s[kMaxRows], m_s[kMaxRows];
   if (a.live_items && (int)blockIdx.x >= *a.live_items) return;
 
-  const WorkItem it = a.items[blockIdx.x];
+  WorkItem it = a.items[blockIdx.x];
   const int kvh = blockIdx.y;
   const int tid = threadIdx.x;
   const int g = a.g;
+  const int q0 = (int)blockIdx.z * (kMaxRows / g);     // this workgroup's queries of the item
+  if (q0 >= it.q_count) return;
+  it.q_begin += q0;
+  it.q_count = min(it.q_count - q0, kMaxRows / g);
+  if (it.out_row >= 0) it.out_row += q0;
+  if (it.vis0 != kNoCausal) it.vis0 += q0;
   const int R = it.q_count * g;
   const T* qbase = reinterpret_cast<const T*>(a.q);
   const T* kv = reinterpret_cast<const T*>(a.kv);
@@ -619,14 +627,28 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
 }
 
 // ================================================================== host: run
+// Whether every row of q, out and the cache starts on 16 bytes, as the MFMA
+// kernels' vector and direct-to-LDS accesses need it.
+static bool rows_aligned(const be_attn_plan_info* info, const AttnArgs& a) {
+  const int64_t es = (int64_t)dtype_size(info->dtype);
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.kv) | reinterpret_cast<uintptr_t>(a.out) |
+                         (uintptr_t)(a.q_sn * es) | (uintptr_t)(a.q_sh * es) | (uintptr_t)(a.o_sn * es) | (uintptr_t)(a.o_sh * es);
+  return (bits & 15) == 0;
+}
+
 template <typename T>
 static int launch_attn(const be_attn_plan_info* info, AttnArgs& a, hipStream_t st) {
-  const dim3 grid(info->grid_items, info->num_kv_heads);
-  if (info->kernel != 0) {
+  // (groups beyond the VALU kernel's rows: vector accesses to q and out take any
+  // alignment, only the direct loads of the cache do not)
+  if (a.g > kMaxRows) BE_REQUIRE((reinterpret_cast<uintptr_t>(a.kv) & 15) == 0, "the cache must be 16-byte aligned");
+  const bool aligned = a.g > kMaxRows || rows_aligned(info, a);
+  const int per = std::max(1, kMaxRows / a.g);         // queries a VALU workgroup takes
+  const dim3 grid(info->grid_items, info->num_kv_heads, (unsigned)ceil_div(std::max(1, info->tile_rows / a.g), per));
+  if (info->kernel != 0 && aligned) {
     if (info->dtype == BE_F32) return fail(BE_ERR_UNSUPPORTED, "MFMA kernel needs fp16/bf16 storage");
     if (info->tile_rows == kMaxTileRows && block_eligible(info->dtype, info->head_dim)) return block_launch(info, a, st);
     return tile_launch(info, a, st);
-  } else if (info->dtype == BE_F32 && info->tile_rows != 0) {
+  } else if (info->dtype == BE_F32 && info->tile_rows != 0 && aligned) {
     return f32_launch(info, a, st);
   } else {
     switch (info->head_dim) {
@@ -662,6 +684,8 @@ int attn_run(const be_attn_plan_info* info, const int32_t* plan, void* partials,
   BE_REQUIRE(info->part_rows_cap == 0 || partials, "plan needs %lld bytes of partial scratch", (long long)info->partial_bytes);
   BE_REQUIRE(info->num_qo_heads % info->num_kv_heads == 0, "corrupt plan info");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const bool worklist = info->kernel < 2 || (info->kernel == 2 && info->stream_loop == kLoopBlocks);
+  BE_REQUIRE(worklist || (reinterpret_cast<uintptr_t>(kv) & 15) == 0, "the cache must be 16-byte aligned");
   if (info->kernel == 2 && info->stream_loop != kLoopBlocks)
     return stream_run(info, plan, partials, q, q_sn, q_sh, kv, out, o_sn, o_sh, lse, sm_scale, phases, st);
   if (info->kernel == 3) return rows_run(info, plan, q, q_sn, q_sh, kv, out, o_sn, o_sh, lse, sm_scale, phases, st);

@@ -269,6 +269,9 @@ typedef struct be_attn_plan_info {
  * KV chunks) and writes the device plan into host_plan[0..info->plan_ints).
  * The caller copies that prefix to device memory (stream-ordered before
  * be_attn_run) and provides info->partial_bytes of device scratch.
+ * Rows of q, out and the cache that do not all start on 16 bytes make be_attn_run
+ * take the VALU kernel on work-list plans (kernel 0, 1 and stream_loop 2); the
+ * other plans refuse them.
  * num_cus sizes the split-K chunking (pass the device's CU count).  caps
  * NULL gives a compact layout sized to this plan; non-NULL the fixed layout
  * above (the fused merge is not available with it). */

@@ -161,6 +161,35 @@ def test_fp32(ws, d, page, rows):
     assert w.stats.kernel == "valu" and w._info.tile_rows in (16, 32, 64)
 
 
+@pytest.mark.parametrize("dtype,n,hq,page,d,fused", [
+    (torch.float32, 40, 8, 16, 128, False), (torch.float32, 5, 8, 3, 64, True), (torch.bfloat16, 70, 16, 8, 128, False),
+    (torch.float16, 300, 16, 16, 128, False), (torch.bfloat16, 9, 8, 8, 256, False), (torch.bfloat16, 30, 8, 16, 64, True)])
+def test_unaligned_cache(ws, dtype, n, hq, page, d, fused):
+    """A cache that starts one element off an allocation: the kernels that load
+    16 bytes a lane, or straight to LDS, leave the work list to the VALU kernel
+    (items of more rows than it holds are shared by its workgroups)."""
+    from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
+    print(f"[case] unaligned cache {dtype} n {n} page {page} d {d}", flush=True)
+    (qo, kvp, kvi, lpl), pages = _levels([n, 3], [n + 900, 40], page)
+    g = torch.Generator().manual_seed(8)
+    kv = torch.randn((pages, 2, page, 2, d), generator=g).to(dtype)
+    q = torch.randn((n + 3, hq, d), generator=g).to(dtype)
+    off = torch.empty(kv.numel() + 1, dtype=dtype, device="cuda")[1:].view(kv.shape)
+    off.copy_(kv)
+    assert off.data_ptr() % 16 != 0 and off.is_contiguous()
+    w = BatchPrefillWithPagedKVCacheWrapper(ws)
+    w._fused_merge, w._tile_kernel, w._num_cus = fused, page % 16 != 0, 8
+    w.plan(qo, kvp, kvi, lpl, hq, 2, d, page, causal=True, q_data_type=dtype)
+    if w._info.kernel == 2 and w._info.stream_loop != 2:
+        with pytest.raises(ValueError, match="aligned"):
+            w.run(q.cuda(), off)
+        return
+    out, lse = w.run(q.cuda(), off, return_lse=True)
+    torch.cuda.synchronize()
+    ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, None, causal=True)
+    _check(out, lse, ref_o, ref_lse, dtype)
+
+
 @pytest.mark.parametrize("tile_rows", [16, 32, 64])
 def test_fp32_fixed_layout(ws, tile_rows):
     """fp32 in a fixed-capacity layout sized for 32-row items."""
