@@ -113,17 +113,17 @@ __device__ void fused_merge_epilogue(const AttnArgs& a, const WorkItem& it, int 
       const int hh = e / D, d = e - hh * D, head = kvh * a.g + hh;
       float M = -INFINITY;
       for (int r = rb; r < re; ++r) M = fmaxf(M, a.part_lse[(int64_t)a.merge_rows[r] * a.hq + head]);
+      const float msafe = M == -INFINITY ? 0.f : M;
       float z = 0.f, acc = 0.f;
-      if (M != -INFINITY) {
-        for (int r = rb; r < re; ++r) {
-          const int64_t row = (int64_t)a.merge_rows[r] * a.hq + head;
-          const float wgt = expf(a.part_lse[row] - M);
-          z += wgt;
-          acc += wgt * a.part_o[row * D + d];
-        }
+      for (int r = rb; r < re; ++r) {
+        const int64_t row = (int64_t)a.merge_rows[r] * a.hq + head;
+        const float wgt = expf(a.part_lse[row] - msafe);
+        z += wgt;
+        // (a row of NaN scores has lse -inf and o NaN: its o counts, with weight 0)
+        acc += wgt * a.part_o[row * D + d];
       }
       T* op = reinterpret_cast<T*>(a.out) + (int64_t)qi * a.o_sn + (int64_t)head * a.o_sh;
-      op[d] = from_f32<T>(z > 0.f ? acc / z : 0.f);
+      op[d] = from_f32<T>(z > 0.f ? acc / z : acc * 0.f);
       if (d == 0 && a.out_lse) a.out_lse[(int64_t)qi * a.hq + head] = (z > 0.f) ? M + logf(z) : -INFINITY;
     }
     if (tid == 0) a.counters[(int64_t)mi * a.hkv + kvh] = 0;

@@ -209,23 +209,31 @@ def test_fp32_fixed_layout(ws, tile_rows):
 
 @pytest.mark.parametrize("dtype,d,page,n", [(torch.bfloat16, 64, 8, 4), (torch.float32, 64, 16, 4), (torch.float32, 128, 16, 4),
                                             (torch.bfloat16, 64, 16, 64)])
-@pytest.mark.parametrize("where", ["k", "v"])
-def test_nan_survives_the_merge(ws, dtype, d, page, n, where):
-    """A NaN key makes every row of its KV head NaN and a NaN value its column,
-    also where the keys are split and the NaN piece is merged with finite ones."""
+@pytest.mark.parametrize("where", ["k", "v", "q"])
+@pytest.mark.parametrize("fused", [False, True])
+def test_nan_survives_the_merge(ws, dtype, d, page, n, where, fused):
+    """A NaN key makes every row of its KV head NaN, a NaN value its column and a
+    NaN query its row, also where the keys are split: the NaN piece is merged with
+    finite ones, or (a query's) every piece is NaN."""
     from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
     print(f"[case] nan {where} d {d} page {page} {dtype}", flush=True)
     (qo, kvp, kvi, lpl), pages = _levels([n], [3000], page)
     g = torch.Generator().manual_seed(5)
     kv = torch.randn((pages, 2, page, 2, d), generator=g).to(dtype)
     q = torch.randn((n, 8, d), generator=g).to(dtype)
-    kv[kvi[1700 // page], 0 if where == "k" else 1, 1700 % page, 1, 7] = math.nan
+    if where == "q":
+        q[2, 5, 7] = math.nan
+    else:
+        kv[kvi[1700 // page], 0 if where == "k" else 1, 1700 % page, 1, 7] = math.nan
     w = BatchPrefillWithPagedKVCacheWrapper(ws)
+    w._fused_merge = fused
     w.plan(qo, kvp, kvi, lpl, 8, 2, d, page, causal=False, q_data_type=dtype)
     out = w.run(q.cuda(), kv.cuda()).float().cpu()
     assert w.stats.num_merge == n and w.stats.kernel != "stream"
     want = torch.zeros_like(out, dtype=torch.bool)
-    if where == "k":
+    if where == "q":
+        want[2, 5] = True
+    elif where == "k":
         want[:, 4:] = True
     else:
         want[:, 4:, 7] = True
