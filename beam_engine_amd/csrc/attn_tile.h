@@ -131,16 +131,20 @@ __device__ void fused_merge_epilogue(const AttnArgs& a, const WorkItem& it, int 
 }
 
 // ---------------------------------------------------------------- tile loads
+static __device__ const uint4 kZeroChunk = {0, 0, 0, 0};
+
 // K and V rows of an item, 64 tokens at a time, global -> LDS directly by the
 // four waves of a workgroup: K at the stage's start, V one plane further, rows of
 // RB bytes whose 16-byte chunk c sits at slot c ^ swz(row).  Load i of wave w
-// moves rows (w IPW + i) RPI .. + RPI - 1 (1 KB of K and 1 KB of V); rows past
-// the item's end re-read its last token (the caller masks them).  Pages and slots
-// advance by whole tiles without a division.
+// moves rows (w IPW + i) RPI .. + RPI - 1 (1 KB of K and 1 KB of V); past the
+// item's end K re-reads its last token (the caller masks the scores) and V reads
+// zeros (a weight of 0 times an infinity would be NaN).  Pages and slots advance
+// by whole tiles without a division.
 //
-// PAGED4: pages hold whole loads' rows (1 KB: 4 tokens of 256-byte rows), so a load's page is wave-uniform: its id comes from a register (64 of the
-// item's ids) by v_readlane, the address is scalar, and a tile's loads cost no
-// vector arithmetic.  Otherwise every lane looks its row's page up in pg_lds
+// PAGED4: pages hold whole loads' rows (1 KB: 4 tokens of 256-byte rows), so a
+// load's page is wave-uniform: its id comes from a register (64 of the item's ids)
+// by v_readlane, the address is scalar, and a whole tile's loads cost no vector
+// arithmetic.  Otherwise every lane looks its row's page up in pg_lds
 // (the caller stages the item's page ids there and synchronises first).
 template <int RB, bool PAGED4, int (*SWZ)(int)>
 struct TileLoader {
@@ -184,6 +188,44 @@ struct TileLoader {
     pg_reg = PAGED4 ? a.pages[it.page_begin + first_page + min(lane, last_page)] : 0;
   }
 
+  // A tile's loads: WHOLE, all its rows lie within the item.
+  template <bool WHOLE>
+  __device__ __forceinline__ void rows(uint32_t dst0) {
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) {
+      const int r0 = (w * IPW + i) * RPI;
+      const uint32_t dst = dst0 + (w * IPW + i) * 1024;
+      const int left = tok_count - 1 - (tok + r0);     // rows of this load up to the last token
+      const bool in = WHOLE || lane / CPR <= left;
+      if constexpr (PAGED4) {
+        const int pg = WHOLE || left >= 0 ? page[i] : last_page, sl = WHOLE || left >= 0 ? slot[i] : last_slot;
+        const int id = __builtin_amdgcn_readlane(pg_reg, pg - pg_base);
+        const uint64_t base = kvb + (uint64_t)((uint32_t)id * 2u * (uint32_t)ps + (uint32_t)sl) * row_bytes;
+        const uint32_t o = (uint32_t)(WHOLE ? lane / CPR : min(lane / CPR, max(left, 0))) * row_bytes + off[i];
+        stream::dma16_sv(base, o, dst);
+        if constexpr (WHOLE) {
+          stream::dma16_sv(base + vplane, o, dst + PLANE);
+        } else {
+          const uint64_t src = base + vplane + o;
+          stream::dma16(in ? reinterpret_cast<const void*>(src) : &kZeroChunk, dst + PLANE);
+        }
+      } else {
+        const uint32_t rec = (uint32_t)pg_lds[in ? page[i] : last_page] * 2u * (uint32_t)ps + (uint32_t)(in ? slot[i] : last_slot);
+        const uint64_t src = kvb + off[i] + (uint64_t)rec * row_bytes;
+        stream::dma16(reinterpret_cast<const void*>(src), dst);
+        stream::dma16(in ? reinterpret_cast<const void*>(src + vplane) : &kZeroChunk, dst + PLANE);
+      }
+      // (a tile that is not whole is the last; with many loads a wave the compiler
+      // makes 6% slower code of leaving the step out there: fp32, head_dim 128)
+      if constexpr (WHOLE || IPW > 4) {
+        slot[i] += dslot;
+        const bool carry = slot[i] >= ps;
+        slot[i] -= carry ? ps : 0;
+        page[i] += dpage + (carry ? 1 : 0);
+      }
+    }
+  }
+
   // The next tile's loads, to LDS byte address dst0 (2 IPW vector memory operations).
   __device__ __forceinline__ void load(uint32_t dst0) {
     if constexpr (PAGED4) {
@@ -194,37 +236,10 @@ struct TileLoader {
         pg_reg = pg_lds[min(pg_base + lane, last_page)];
       }
     }
-    const bool whole = tok + kTile <= tok_count;         // uniform
-#pragma unroll
-    for (int i = 0; i < IPW; ++i) {
-      const int r0 = (w * IPW + i) * RPI;
-      const uint32_t dst = dst0 + (w * IPW + i) * 1024;
-      if constexpr (PAGED4) {
-        int pg = page[i], sl = slot[i], lr = lane / CPR;
-        if (!whole) {
-          const int left = tok_count - 1 - (tok + r0);   // rows of this load up to the last token
-          if (left < 0) {
-            pg = last_page;
-            sl = last_slot;
-          }
-          lr = min(lr, max(left, 0));
-        }
-        const int id = __builtin_amdgcn_readlane(pg_reg, pg - pg_base);
-        const uint64_t base = kvb + (uint64_t)((uint32_t)id * 2u * (uint32_t)ps + (uint32_t)sl) * row_bytes;
-        const uint32_t o = (uint32_t)lr * row_bytes + off[i];
-        stream::dma16_sv(base, o, dst);
-        stream::dma16_sv(base + vplane, o, dst + PLANE);
-      } else {
-        const bool in = whole || tok + r0 + lane / CPR < tok_count;
-        const uint32_t rec = (uint32_t)pg_lds[in ? page[i] : last_page] * 2u * (uint32_t)ps + (uint32_t)(in ? slot[i] : last_slot);
-        const uint64_t src = kvb + off[i] + (uint64_t)rec * row_bytes;
-        stream::dma16(reinterpret_cast<const void*>(src), dst);
-        stream::dma16(reinterpret_cast<const void*>(src + vplane), dst + PLANE);
-      }
-      slot[i] += dslot;
-      const bool carry = slot[i] >= ps;
-      slot[i] -= carry ? ps : 0;
-      page[i] += dpage + (carry ? 1 : 0);
+    if (__builtin_expect(tok + kTile <= tok_count, 1)) {
+      rows<true>(dst0);
+    } else {
+      rows<false>(dst0);
     }
     tok += kTile;
   }

@@ -207,6 +207,31 @@ def test_fp32_fixed_layout(ws, tile_rows):
     _check(out, lse, ref_o, ref_lse, torch.float32)
 
 
+@pytest.mark.parametrize("dtype,d,page,n,hq", [
+    (torch.float32, 64, 16, 2, 8), (torch.float32, 128, 3, 8, 8), (torch.float32, 256, 8, 30, 8), (torch.bfloat16, 64, 8, 2, 8),
+    (torch.bfloat16, 256, 3, 20, 8), (torch.float16, 128, 8, 8, 8), (torch.float16, 64, 16, 40, 8), (torch.bfloat16, 128, 5, 90, 8)])
+@pytest.mark.parametrize("kv_len", [1, 63, 70, 127, 200])
+def test_infinite_value_of_the_last_token(ws, dtype, d, page, n, hq, kv_len):
+    """An infinite value element of a group's last token makes its column
+    infinite: what fills the token tile beyond the group's end does not meet it
+    (0 x infinity)."""
+    from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
+    print(f"[case] inf d {d} page {page} {dtype} n {n} kv {kv_len}", flush=True)
+    (qo, kvp, kvi, lpl), pages = _levels([n], [kv_len], page)
+    g = torch.Generator().manual_seed(5)
+    kv = torch.randn((pages, 2, page, 2, d), generator=g).to(dtype)
+    kv[kvi[(kv_len - 1) // page], 1, (kv_len - 1) % page, 1, 7] = math.inf
+    q = torch.randn((n, hq, d), generator=g).to(dtype)
+    w = BatchPrefillWithPagedKVCacheWrapper(ws)
+    w._tile_kernel = True
+    w.plan(qo, kvp, kvi, lpl, hq, 2, d, page, causal=False, q_data_type=dtype)
+    out = w.run(q.cuda(), kv.cuda()).float().cpu()
+    assert not out.isnan().any()
+    want = torch.zeros_like(out, dtype=torch.bool)
+    want[:, hq // 2:, 7] = True
+    assert torch.equal(out == math.inf, want)
+
+
 @pytest.mark.parametrize("dtype,d,page,n", [(torch.bfloat16, 64, 8, 4), (torch.float32, 64, 16, 4), (torch.float32, 128, 16, 4),
                                             (torch.bfloat16, 64, 16, 64)])
 @pytest.mark.parametrize("where", ["k", "v", "q"])
