@@ -385,13 +385,47 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
     info->flops = flops;
     return BE_OK;
   }
-  // causal groups of enough query rows run as 128-row blocks instead
   const int q_tile = std::max(1, rows_cap / g);
-  int64_t causal_blocks = 0;
-  for (const Group& gr : groups)
-    if (gr.kv_len > 0 && is_causal(gr)) causal_blocks += ceil_div(gr.q1 - gr.q0, q_tile) * hkv;
+  // Causal groups on the block kernel: a workgroup's tiles run one after the
+  // other (about 1.5 us each with the CU to itself, 1.05 us per tile of the CU's
+  // two workgroups together: head_dim 128, MI355X), and splitting their keys costs
+  // the merge pass (about 8 us) and the fp32 partials' round trip.  The longest
+  // query tile is cut into the number of chunks, a power of two, that makes the
+  // slower of its own chain and the CUs' shares shortest, those costs included
+  // (1000 fresh tokens, 32 / 8 heads: two chunks take 14% longer than whole).
+  int64_t causal_chunk = 0, causal_blocks = 0, tiles = 0, queries = 0, span = 0;
+  double block_us = 0;
+  if (any_causal && mfma && !less && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
+    int64_t longest = 0;
+    for (const Group& gr : groups) {
+      if (gr.kv_len <= 0 || gr.q1 <= gr.q0) continue;
+      if (is_causal(gr)) causal_blocks += ceil_div(gr.q1 - gr.q0, q_tile) * hkv;
+      queries += gr.q1 - gr.q0;
+      span = std::max<int64_t>(span, gr.q1 - gr.q0);
+      for (int qa = gr.q0; qa < gr.q1; qa += q_tile) {
+        const int64_t t = ceil_div(vis(gr, std::min(qa + q_tile, gr.q1) - 1), kTile);
+        longest = std::max(longest, t);
+        tiles += t * hkv;
+      }
+    }
+    const double per_d = 0.3 + 0.7 * d / 128;        // a tile's time against head_dim 128
+    for (int64_t cut = 1; cut == 1 || longest / cut >= 8; cut *= 2) {
+      const int64_t c = ceil_div(longest, cut);
+      double t = per_d * std::max(1.5 * c, 1.05 * tiles / num_cus);
+      if (cut > 1) t += 8.0 + 2.0 * cut * queries * hq * d * 4 / 5e6;
+      if (cut == 1 || t < block_us) {
+        block_us = t;
+        causal_chunk = c * kTile;
+      }
+    }
+  }
+  // causal groups of enough query rows run as 128-row blocks rather than on the
+  // streaming kernel, unless its even shares of the same tiles and its merge of
+  // 16-bit slots take less
   const bool streams = stream_eligible(dtype, d, g, page_size, flags);
-  const bool blocks = streams && !caps && !less && !(flags & BE_PLAN_NO_BLOCKS) && causal_blocks >= kMinCausalBlocks;
+  const bool blocks = streams && !caps && !less && !(flags & BE_PLAN_NO_BLOCKS) && causal_blocks >= kMinCausalBlocks &&
+                      block_us <= kStreamUs + kStreamTileUs * tiles / num_cus + kStreamRowUs * queries * hq +
+                                      kStreamSpanUs * span / kTile;
   if (!(any_causal && caps) && streams && !blocks && (!caps || caps->tile_rows == 64)) {
     memset(info, 0, sizeof(*info));
     const int rc = stream_plan(groups, levels, num_levels, total_pages, num_queries, hq, hkv, d, page_size,
@@ -424,38 +458,6 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   // an item's page ids are staged in LDS: at most kMaxPagesLds pages per item
   const int64_t chunk_cap = std::max<int64_t>(64, ((int64_t)(kMaxPagesLds - 1) * page_size) / 64 * 64);
   if (chunk > chunk_cap) chunk = chunk_cap;
-
-  // Causal groups on the block kernel: a workgroup's tiles run one after the
-  // other (about 1.5 us each with the CU to itself, 1.05 us per tile of the CU's
-  // two workgroups together: head_dim 128, MI355X), and splitting their keys costs
-  // the merge pass (about 8 us) and the fp32 partials' round trip.  The longest
-  // query tile is cut into the number of chunks, a power of two, that makes the
-  // slower of its own chain and the CUs' shares shortest, those costs included
-  // (1000 fresh tokens, 32 / 8 heads: two chunks take 14% longer than whole).
-  int64_t causal_chunk = 0;
-  if (any_causal && mfma && !less && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
-    int64_t longest = 0, total = 0, queries = 0;
-    for (const Group& gr : groups) {
-      if (gr.kv_len <= 0 || gr.q1 <= gr.q0) continue;
-      queries += gr.q1 - gr.q0;
-      for (int qa = gr.q0; qa < gr.q1; qa += q_tile) {
-        const int64_t t = ceil_div(vis(gr, std::min(qa + q_tile, gr.q1) - 1), kTile);
-        longest = std::max(longest, t);
-        total += t * hkv;
-      }
-    }
-    const double per_d = 0.3 + 0.7 * d / 128;        // a tile's time against head_dim 128
-    double best = 0;
-    for (int64_t cut = 1; cut == 1 || longest / cut >= 8; cut *= 2) {
-      const int64_t c = ceil_div(longest, cut);
-      double t = per_d * std::max(1.5 * c, 1.05 * total / num_cus);
-      if (cut > 1) t += 8.0 + 2.0 * cut * queries * hq * d * 4 / 5e6;
-      if (cut == 1 || t < best) {
-        best = t;
-        causal_chunk = c * kTile;
-      }
-    }
-  }
 
   // A chunk of a group writes rows x D x 4 bytes of partials per KV head while
   // reading 4 x D bytes per token (bf16 K + V): keep chunks >= 4 x rows tokens

@@ -266,6 +266,15 @@ constexpr int kLoopBlocks = 2;
 // 243.6 -> 112; 8 x 1024 tokens 252 -> 103; 8 / 8 heads, 1000 tokens (64 blocks)
 // about even.
 constexpr int64_t kMinCausalBlocks = 64;
+// The streaming kernel's time beyond the block kernel's fixed one: a constant, a
+// 128-row x 64-token tile of a CU's share, a (query, head) row, 64 new tokens of the
+// longest prompt.  Few new tokens after some cached ones leave too few blocks, each
+// a long chain: 256 after 400 cached, 32 / 8 heads, 17.7 us streaming against 20.8,
+// 512 after 400, 16 / 4 heads, 19.9 against 26.0; 2 x 256 after 8000, whose keys are
+// split, 190 against 90.  Fitted to 426 plans (1 to 16 prompts of 16 to 4096 new
+// tokens after 0 to 30000 cached ones, 4 to 128 query heads): by the block count
+// alone 22 of them took up to 29% longer than on the other kernel, now 3 do, up to 7%.
+constexpr double kStreamUs = 1.5, kStreamTileUs = 3.8, kStreamRowUs = 4e-4, kStreamSpanUs = 0.5;
 
 // True when the block kernel has an instantiation for this shape.
 bool block_eligible(int dtype, int head_dim);

@@ -642,6 +642,20 @@ def test_causal_block_plan_covers_visible_tokens(q_lens, cached, hq, hkv, cus):
     assert rc == 0 and (info.kernel, info.stream_loop) != (2, 2)
 
 
+@pytest.mark.parametrize("reqs,n,cached,hq,hkv,blocks", [
+    (1, 256, 0, 32, 8, True), (1, 256, 400, 32, 8, False), (1, 512, 400, 16, 4, False), (2, 256, 8000, 32, 8, True),
+    (8, 1024, 0, 32, 8, True), (1, 3000, 0, 8, 1, True), (16, 32, 0, 32, 8, True)])
+def test_causal_plans_take_the_faster_kernel(reqs, n, cached, hq, hkv, blocks):
+    """Blocks or the streaming kernel by their modelled times, not by the number
+    of blocks alone: a few new tokens after some cached ones stay streaming."""
+    npg = -(-(n + cached) // 16)
+    levels = [([i * n for i in range(reqs + 1)], [i * npg for i in range(reqs + 1)], list(range(reqs * npg)),
+               [n + cached - (npg - 1) * 16] * reqs)]
+    rc, info, _, _, L = plan(levels, hq=hq, hkv=hkv, page=16, num_pages=reqs * npg, flags=128)
+    assert rc == 0, L.be_last_error()
+    assert info.kernel == 2 and (info.stream_loop == 2) == blocks
+
+
 @pytest.mark.parametrize("d,page,tokens,dtype,fits", [(128, 16, 1000, 0, 12_544), (128, 32, 1000, 0, 12_288)])
 def test_less_scratch_fp32_plan(d, page, tokens, dtype, fits):
     """fp32 prompts on 64-row items are cut into more key splits than on 32-row
