@@ -393,19 +393,30 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   // query tile is cut into the number of chunks, a power of two, that makes the
   // slower of its own chain and the CUs' shares shortest, those costs included
   // (1000 fresh tokens, 32 / 8 heads: two chunks take 14% longer than whole).
+  // Plans of at most 64 rows an item run on the tile kernel instead, in tiles of
+  // half the time before a merge of few rows: where that cut leaves half the CUs
+  // idle it is halved until they have a workgroup each, down to two tiles or to 16
+  // chunks, whose merge is two batches (4 new tokens after 3000, 8 / 8 heads,
+  // head_dim 128, page 8: 16.7 us at 4 chunks, 11.2 at 16) -- whole tiles only from
+  // about 6 us, what the merge pass takes (16 after 400, head_dim 64, 7.3 us whole,
+  // 9.4 in 4 chunks; after 1000 11.8 and 9.2).
   int64_t causal_chunk = 0, causal_blocks = 0, tiles = 0, queries = 0, span = 0;
   double block_us = 0;
   if (any_causal && mfma && !less && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
     int64_t longest = 0;
+    int most_rows = 0;
+    std::vector<int64_t> tiles_of;                     // of each query tile
     for (const Group& gr : groups) {
       if (gr.kv_len <= 0 || gr.q1 <= gr.q0) continue;
       if (is_causal(gr)) causal_blocks += ceil_div(gr.q1 - gr.q0, q_tile) * hkv;
       queries += gr.q1 - gr.q0;
+      most_rows = std::max(most_rows, std::min(q_tile, gr.q1 - gr.q0) * g);
       span = std::max<int64_t>(span, gr.q1 - gr.q0);
       for (int qa = gr.q0; qa < gr.q1; qa += q_tile) {
         const int64_t t = ceil_div(vis(gr, std::min(qa + q_tile, gr.q1) - 1), kTile);
         longest = std::max(longest, t);
         tiles += t * hkv;
+        tiles_of.push_back(t);
       }
     }
     const double per_d = 0.3 + 0.7 * d / 128;        // a tile's time against head_dim 128
@@ -417,6 +428,13 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
         block_us = t;
         causal_chunk = c * kTile;
       }
+    }
+    const bool cut_more = most_rows <= 64 && (causal_chunk < longest * kTile || 0.7 * per_d * longest > 6.0);
+    for (int64_t c = causal_chunk / kTile; cut_more && c > 2; c = ceil_div(c, 2)) {
+      int64_t wgs = 0;
+      for (int64_t t : tiles_of) wgs += ceil_div(t, c) * hkv;
+      if (2 * wgs > num_cus || ceil_div(longest, ceil_div(c, 2)) > 16) break;
+      causal_chunk = ceil_div(c, 2) * kTile;
     }
   }
   // causal groups of enough query rows run as 128-row blocks rather than on the

@@ -656,6 +656,22 @@ def test_causal_plans_take_the_faster_kernel(reqs, n, cached, hq, hkv, blocks):
     assert info.kernel == 2 and (info.stream_loop == 2) == blocks
 
 
+@pytest.mark.parametrize("reqs,n,cached,hq,hkv,d,page,items", [
+    (1, 4, 3000, 8, 8, 128, 8, 16), (1, 16, 400, 8, 8, 64, 16, 1), (1, 16, 1000, 8, 8, 64, 16, 8), (1, 2, 20000, 8, 8, 128, 8, 32),
+    (16, 8, 400, 32, 8, 128, 8, 16)])
+def test_causal_tile_plans_fill_the_chip(reqs, n, cached, hq, hkv, d, page, items):
+    """Causal plans of at most 64 rows an item (the tile kernel): cut until half the
+    CUs have a workgroup, whole where they are short or the CUs are busy."""
+    npg = -(-(n + cached) // page)
+    levels = [([i * n for i in range(reqs + 1)], [i * npg for i in range(reqs + 1)], list(range(reqs * npg)),
+               [n + cached - (npg - 1) * page] * reqs)]
+    rc, info, buf, _, L = plan(levels, hq=hq, hkv=hkv, d=d, page=page, num_pages=reqs * npg, flags=128)
+    assert rc == 0, L.be_last_error()
+    assert info.kernel == 1 and info.tile_rows <= 64 and info.num_items == items
+    it = decode_items(info, buf)
+    assert it[:, 4].sum() == reqs * (n + cached) and (it[:, 3] % 64 == 0).all()
+
+
 @pytest.mark.parametrize("d,page,tokens,dtype,fits", [(128, 16, 1000, 0, 12_544), (128, 32, 1000, 0, 12_288)])
 def test_less_scratch_fp32_plan(d, page, tokens, dtype, fits):
     """fp32 prompts on 64-row items are cut into more key splits than on 32-row
