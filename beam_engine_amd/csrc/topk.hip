@@ -66,13 +66,21 @@ struct TopkGeom {
 // often, and the row pass merges more lists.
 constexpr int kMinSegLen = 2048;
 constexpr int kSplitRowCand = 2048;  // segs x cap of a row split for parallelism: two candidates per pass-B thread
+// Short rows, k above 16: up to this many segments where every position then fits
+// the candidate space (no threshold to search, none to overflow).  MI355X, us per
+// call, as one segment and so: 64 rows x 600 fp32, k 32, 36.4 and 29.9; 32 rows x 2000
+// fp32, k 64, 77.0 and 63.8 (bf16 31.8 and 35.9); 64 rows x 1000 bf16, k 32, 28.3 and
+// 22.9.
+constexpr int kShortSegs = 8;
 
 static TopkGeom topk_geom(int n_rows, int vocab, int k) {
   int segs = (vocab + kMaxSegLen - 1) / kMaxSegLen;
   // few rows: up to about two workgroups per CU, as long as a segment keeps
   // kMinSegLen logits and pass B two candidates per thread
   int want = (512 + n_rows - 1) / n_rows;
+  const int brief = std::min(want, kShortSegs);
   want = std::min(want, std::min(vocab / kMinSegLen, kSplitRowCand / topk_cap(k)));
+  if (topk_cap(k) > 64 && vocab <= brief * topk_cap(k)) want = brief;
   if (want > segs) segs = want;
   const int by_k = (vocab + k - 1) / k;                   // every segment holds >= k elements
   if (segs > by_k) segs = by_k;

@@ -315,7 +315,8 @@ def test_pool_bound_and_full_ranking():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("n,v,beam", [(1, 7, 1), (1, 5, 2), (2, 1021, 4), (3, 257, 8), (2, 2047, 16), (4, 4100, 4), (1, 6145, 32),
-                                      (2, 10007, 2), (4, 32000, 4), (8, 128256, 8), (2, 70001, 64)])
+                                      (2, 10007, 2), (4, 32000, 4), (8, 128256, 8), (2, 70001, 64), (64, 1024, 16),
+                                      (64, 1025, 16), (128, 512, 16), (5, 2048, 32), (5, 2049, 32), (2, 300, 64), (200, 200, 16)])
 def test_few_rows_and_short_segments(dtype, n, v, beam):
     """Few rows (split into segments no shorter than a chunk per thread) and
     vocabularies that leave waves of a segment partly or wholly without
