@@ -83,7 +83,10 @@ def _num_cus(device: torch.device) -> int:
 
 
 class PlanStats:
-    """Algorithmic work of a plan (for roofline reporting)."""
+    """Algorithmic work of a plan (for roofline reporting).  ``kernel`` is the plan
+    kind; ``launches`` names the device kernels of a run (a "stream" plan whose
+    causal groups run as 128-row blocks launches attn_block_kernel, a "valu" one
+    in fp32 attn_f32_kernel)."""
 
     def __init__(self, info: _lib.BeAttnPlanInfo):
         self.kv_bytes = int(info.kv_bytes)
@@ -95,6 +98,18 @@ class PlanStats:
         self.kernel = {0: "valu", 1: "tile", 2: "stream", 3: "rows"}[int(info.kernel)]
         self.num_tails = int(info.num_tails) if self.kernel == "stream" else 0
         self.chunk_tokens = int(info.chunk_tokens)
+        merge = (int(info.grid_merge) > 0 and not info.fused_merge) or int(info.grid_zero) > 0
+        if self.kernel == "rows":
+            self.launches = ("attn_rows_kernel",)
+        elif self.kernel == "stream" and info.stream_loop != 2:
+            self.launches = ("attn_stream_kernel",) + (("tail_merge_kernel",) if info.grid_merge > 0 else ())
+        else:
+            rows = int(info.tile_rows)
+            if info.kernel == 0:
+                name = "attn_f32_kernel" if rows and info.dtype == _lib.dtype_code(torch.float32) else "attn_valu_kernel"
+            else:
+                name = "attn_block_kernel" if rows == 128 and int(info.head_dim) <= 128 else "attn_tile_kernel"
+            self.launches = (name,) + (("merge_kernel",) if merge else ())
 
     @property
     def bytes(self) -> int:

@@ -619,7 +619,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   info->kernel = blocks ? 2 : mfma ? 1 : 0;
   info->stream_loop = blocks ? kLoopBlocks : 0;
   info->tile_rows = !mfma && !f32 ? 0 : blocks ? 128 : caps ? (f32 ? rows_cap : caps->tile_rows) : (max_r <= 16 ? 16 : max_r <= 32 ? 32 : max_r <= 64 ? 64 : 128);
-  info->chunk_tokens = (int32_t)std::min<int64_t>(chunk, INT32_MAX);
+  info->chunk_tokens = (int32_t)std::min<int64_t>(causal_chunk > 0 ? std::min(causal_chunk, chunk_cap) : chunk, INT32_MAX);
   info->plan_ints = (int32_t)off;
   info->off_items = (int32_t)off_items;
   info->off_qindex = (int32_t)off_qindex;

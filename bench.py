@@ -163,8 +163,7 @@ def attention_workload(args):
     traffic, traffic_src = attention_traffic(wl.name, args)
     roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_src,
-            "kernel": f"attn_{st.kernel}_kernel" + ("" if st.num_merge == 0 or args.fused_merge else
-                                                    " + tail_merge_kernel" if st.kernel == "stream" else " + merge_kernel"),
+            "kernel": " + ".join(st.launches),
             "bytes_per_launch": alg, "mean_launch_us": round(mean_us, 2), "median_launch_us": round(med_us, 2),
             "tflops": round(tflops, 2), "mfma_frac": round(tflops / BF16_PEAK_TFLOPS, 4)}
     result = {
@@ -227,8 +226,7 @@ def prefill_workload(args):
                    "layers": L, "items": st.num_items, "flops_per_launch": st.flops},
         "roofline": {"bound": "mfma", "achieved": round(tflops, 2), "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / BF16_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": f"attn_{st.kernel}_kernel" + (" + tail_merge_kernel" if st.kernel == "stream" else
-                                                             " + merge_kernel"),
+                     "kernel": " + ".join(st.launches),
                      "mean_launch_us": round(mean_us, 2),
                      "hbm_gbs": round(gbs, 1)},
     }

@@ -116,7 +116,7 @@ class AttnTimer:
 
     def _bytes(self, wrapper):
         st = wrapper.stats
-        self.kernels.add(st.kernel)
+        self.kernels.add(" + ".join(st.launches))
         if self.kind == "flat":
             # the flat strategy is scored by its own traffic: every query's whole path
             hq = wrapper._info.num_qo_heads
@@ -396,9 +396,7 @@ def run_e2e_bench(args):
         "roofline": {"bound": "hbm", "achieved": round(att["gbs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(att["gbs"] / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": traffic_src,
-                     "kernel": " / ".join(f"attn_{k}_kernel" for k in kern) +
-                               (" + tail_merge_kernel" if kern == ["stream"] else " + merge_kernel") +
-                               " (decode attention: both kernels of a launch)",
+                     "kernel": " / ".join(kern) + " (decode attention: the kernels of a launch)",
                      "timed_launches": att["launches"],
                      "timed_sample": "the launch of layer (step mod 32) in every timed step",
                      "bytes_per_launch": round(att["bytes_per_launch"]),

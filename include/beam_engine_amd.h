@@ -216,10 +216,14 @@ typedef struct be_attn_plan_info {
   int32_t num_merge;       /* queries merged by the merge kernel               */
   int32_t num_queries;
   int32_t num_qo_heads, num_kv_heads, head_dim, page_size, num_pages, dtype;
-  int32_t kernel;          /* 0 = fp32 (MFMA; tile_rows 0: VALU), 1 = MFMA tile, 2 = MFMA streaming (persistent),
-                              3 = MFMA row blocks (one kernel, no merge)           */
-  int32_t tile_rows;       /* rows (queries x GQA group) per MFMA tile: 16/32  */
-  int32_t chunk_tokens;    /* split-K chunk length                             */
+  int32_t kernel;          /* 0 = work list on the fp32 MFMA kernel (tile_rows 0: VALU),
+                              1 = work list on the 16-bit MFMA tile kernel (tile_rows 128:
+                              the block kernel), 2 = MFMA streaming (persistent; stream_loop 2:
+                              a work list on the block kernel), 3 = MFMA row blocks (one
+                              kernel, no merge)                                    */
+  int32_t tile_rows;       /* most rows (queries x GQA group) of an item: 16, 32, 64, 128 */
+  int32_t chunk_tokens;    /* split-K chunk length (fewer-row groups of non-causal plans
+                              may take longer ones)                               */
   int32_t plan_ints;       /* int32 words of the device plan                    */
   int32_t off_items, off_qindex, off_pages, off_merge_q, off_merge_ptr, off_merge_rows;
   int32_t off_q_merge;     /* per query: index into the merge list, or -1      */

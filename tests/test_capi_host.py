@@ -672,6 +672,25 @@ def test_causal_tile_plans_fill_the_chip(reqs, n, cached, hq, hkv, d, page, item
     assert it[:, 4].sum() == reqs * (n + cached) and (it[:, 3] % 64 == 0).all()
 
 
+@pytest.mark.parametrize("dtype,d,page,n,cached,flags,launches,chunk", [
+    (2, 128, 16, 1000, 0, 128, ("attn_block_kernel",), 1024), (2, 128, 16, 256, 8000, 128, ("attn_block_kernel", "merge_kernel"), None),
+    (2, 128, 16, 1000, 0, 128 | 4096, ("attn_stream_kernel", "tail_merge_kernel"), None),
+    (1, 128, 8, 1000, 0, 128, ("attn_block_kernel",), 1024), (1, 128, 8, 4, 300, 128, ("attn_tile_kernel",), 320),
+    (2, 256, 16, 40, 0, 128, ("attn_tile_kernel",), None), (0, 128, 16, 40, 0, 128, ("attn_f32_kernel",), None),
+    (0, 128, 16, 40, 0, 129, ("attn_valu_kernel",), None), (2, 128, 16, 1, 2000, 256, ("attn_rows_kernel",), None)])
+def test_plan_stats_name_the_kernels_that_run(dtype, d, page, n, cached, flags, launches, chunk):
+    """PlanStats.launches names the device kernels of a run, chunk_tokens the
+    chunks they were given (causal cuts included)."""
+    from beam_engine_amd.attention import PlanStats
+    npg = -(-(n + cached) // page)
+    levels = [([0, n], [0, npg], list(range(npg)), [n + cached - (npg - 1) * page])]
+    rc, info, _, _, L = plan(levels, hq=32, hkv=8, d=d, page=page, num_pages=npg, dtype=dtype, flags=flags)
+    assert rc == 0, L.be_last_error()
+    st = PlanStats(info)
+    assert st.launches == launches
+    assert chunk is None or st.chunk_tokens == chunk
+
+
 @pytest.mark.parametrize("d,page,tokens,dtype,fits", [(128, 16, 1000, 0, 12_544), (128, 32, 1000, 0, 12_288)])
 def test_less_scratch_fp32_plan(d, page, tokens, dtype, fits):
     """fp32 prompts on 64-row items are cut into more key splits than on 32-row
