@@ -22,7 +22,7 @@ def ws():
     return torch.empty(256 << 20, dtype=torch.uint8, device="cuda")
 
 
-def _run(ws, dtype, q_lens, kv_lens, hq, hkv, d, page, causal=True, sm_scale=None, shuffle=3, cus=None):
+def _run(ws, dtype, q_lens, kv_lens, hq, hkv, d, page, causal=True, sm_scale=None, shuffle=3, cus=None, kernel=None):
     from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
     (qo, kvp, kvi, lpl), pages = _levels(q_lens, kv_lens, page)
     g = torch.Generator().manual_seed(shuffle)
@@ -32,6 +32,7 @@ def _run(ws, dtype, q_lens, kv_lens, hq, hkv, d, page, causal=True, sm_scale=Non
     w = BatchPrefillWithPagedKVCacheWrapper(ws)
     w._num_cus = cus
     w.plan(qo, kvp, kvi, lpl, hq, hkv, d, page, causal=causal, sm_scale=sm_scale, q_data_type=dtype)
+    assert kernel is None or w.stats.launches[0] == kernel
     out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
     torch.cuda.synchronize()
     ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, sm_scale, causal=causal)
@@ -45,9 +46,14 @@ def _run(ws, dtype, q_lens, kv_lens, hq, hkv, d, page, causal=True, sm_scale=Non
 def test_pages_and_head_dims(ws, dtype, page, d):
     """Page sizes that hold whole load groups (4 rows at head_dim 128, 8 at 64)
     and ones that do not, prompts around the 32-query block and 64-token tile,
-    with cached tokens before them."""
+    with cached tokens before them (longer ones where the streaming kernel, which
+    takes head_dim 128 on pages of 16, would run few blocks)."""
     print(f"[case] block page {page} d {d} {dtype}", flush=True)
-    _run(ws, dtype, [33, 129, 64], [33, 200, 65], 16, 4, d, page)
+    if d == 128 and page % 16 == 0:
+        q_lens, kv_lens = [65, 290, 128], [65, 361, 129]
+    else:
+        q_lens, kv_lens = [33, 129, 64], [33, 200, 65]
+    _run(ws, dtype, q_lens, kv_lens, 16, 4, d, page, kernel="attn_block_kernel")
 
 
 @pytest.mark.parametrize("hq,hkv", [(8, 8), (12, 4), (40, 8), (64, 2), (48, 1), (128, 1)])
@@ -55,7 +61,7 @@ def test_group_sizes(ws, hq, hkv):
     """GQA groups that divide the 128-row block and ones that leave rows unused."""
     print(f"[case] block group {hq}/{hkv}", flush=True)
     n = 140 if hq // hkv < 32 else 12
-    _run(ws, torch.bfloat16, [n], [n + 77], hq, hkv, 64, 16)
+    _run(ws, torch.bfloat16, [n], [n + 77], hq, hkv, 64, 16, kernel="attn_block_kernel")
 
 
 @pytest.mark.parametrize("causal", [True, False])
@@ -64,7 +70,7 @@ def test_scales_and_unmasked(ws, causal, scale):
     """Any sign of the scale (the block softmax takes the max of unscaled
     scores), masked and unmasked."""
     print(f"[case] block scale {scale} causal {causal}", flush=True)
-    _run(ws, torch.bfloat16, [70, 5], [70, 130], 32, 8, 64, 8, causal=causal, sm_scale=scale)
+    _run(ws, torch.bfloat16, [70, 5], [70, 130], 32, 8, 64, 8, causal=causal, sm_scale=scale, kernel="attn_block_kernel")
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
@@ -76,17 +82,40 @@ def test_few_rows(ws, d, page, rows):
     ids, causal, at every head_dim."""
     n, g = rows
     print(f"[case] tile rows {n} x {g} d {d} page {page}", flush=True)
-    _run(ws, torch.bfloat16, [n, n, n], [63, 130, 400], 2 * g, 2, d, page)
+    # (head_dim 128 on pages of 16 streams)
+    _run(ws, torch.bfloat16, [n, n, n], [63, 130, 400], 2 * g, 2, d, page,
+         kernel=None if d == 128 and page == 16 else "attn_tile_kernel")
 
 
 @pytest.mark.parametrize("page", [1, 4, 16])
 def test_keys_split_over_blocks(ws, page):
-    """Few queries over many cached tokens: the keys are cut into chunks (several
-    windows of 64 page ids each) and merged; page 1 also meets the page-id limit
-    of one item."""
+    """Few queries over many cached tokens: the keys are cut into chunks and
+    merged; page 1 also meets the page-id limit of one item."""
     print(f"[case] block split page {page}", flush=True)
-    w = _run(ws, torch.float16, [40], [3000], 32, 8, 64, page)
+    w = _run(ws, torch.float16, [40], [3000], 32, 8, 64, page, kernel="attn_block_kernel")
     assert w.stats.num_merge == 40
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("q_lens,kv_lens,page", [([256], [8256], 16), ([100, 40], [4000, 3000], 8), ([70], [2000], 5)])
+def test_keys_split_over_blocks_d128(ws, dtype, q_lens, kv_lens, page):
+    """The same at head_dim 128: partial rows of several chunks per query, on
+    plans of both kinds that run blocks, and the merge."""
+    print(f"[case] block split d128 page {page} {dtype}", flush=True)
+    w = _run(ws, dtype, q_lens, kv_lens, 32, 8, 128, page, kernel="attn_block_kernel")
+    assert w.stats.num_merge == sum(q_lens) and w.stats.launches == ("attn_block_kernel", "merge_kernel")
+    assert (w._info.kernel, w._info.stream_loop) == ((2, 2) if page == 16 else (1, 0))
+
+
+@pytest.mark.parametrize("d,page,n,kv_len", [(128, 4, 70, 1400), (128, 8, 70, 2500), (64, 8, 70, 2500), (128, 8, 600, 4000),
+                                             (128, 1, 70, 900), (128, 12, 70, 2000)])
+def test_long_items(ws, d, page, n, kv_len):
+    """Items of hundreds of pages (one CU: the keys stay whole): where pages hold
+    whole load groups the page ids pass through windows of 64, elsewhere every
+    lane looks its row's up."""
+    print(f"[case] block windows d {d} page {page}", flush=True)
+    w = _run(ws, torch.bfloat16, [n], [kv_len], 32, 8, d, page, cus=1, kernel="attn_block_kernel")
+    assert w.stats.num_merge == 0 and kv_len // page > 128
 
 
 @pytest.mark.parametrize("dtype,hq,hkv,page,n,kv_len,small", [
@@ -159,6 +188,7 @@ def test_fp32(ws, d, page, rows):
     print(f"[case] f32 rows {n} x {g} d {d} page {page}", flush=True)
     w = _run(ws, torch.float32, [n, n, 1], [64, 131, 390], 2 * g, 2, d, page)
     assert w.stats.kernel == "valu" and w._info.tile_rows in (16, 32, 64)
+    assert w.stats.launches[0] == "attn_f32_kernel"
 
 
 @pytest.mark.parametrize("dtype,n,hq,page,d,fused", [

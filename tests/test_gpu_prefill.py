@@ -5,8 +5,10 @@ and causal=True (models/modeling_llama.py:213-283, 775-798).  Cases: fresh
 prompts (queries == keys), prompts continuing cached tokens (fewer queries
 than keys), more queries than keys (the first see nothing: o = 0, lse =
 -inf), ragged batches, GQA groups 1/4/8, head_dim 64/128, page sizes 4/16,
-fp32 (1e-5) and bf16 / fp16 (2e-2 rel, 1e-2 abs), few CUs (many chunks and
-partial rows), and causal multi-query groups on a cascade's last level."""
+fp32 (1e-5) and bf16 / fp16 (2e-2 rel, 1e-2 abs), few CUs (long runs and
+whole items), the streaming kernel where blocks are the default (what a small
+workspace falls back to), and causal multi-query groups on a cascade's last
+level."""
 
 import math
 
@@ -59,7 +61,7 @@ CASES = {
     "more_queries_than_keys": ([8], [5], 8, 8, 128, 4),
     "g8_page4": ([129, 77], [129, 200], 64, 8, 128, 4),
     "mha_d64": ([96, 31], [96, 31], 8, 8, 64, 16),
-    # a long prompt at every storage type, fp32 included (the VALU kernel's long causal path)
+    # a long prompt at every storage type, fp32 included
     "long_mha_d64": ([1000], [1000], 8, 8, 64, 16),
 }
 
@@ -81,14 +83,44 @@ def test_prefill_wrapper_causal(ws, dtype, case, cus):
     w.plan(torch.tensor(qo, dtype=torch.int32), torch.tensor(kvp, dtype=torch.int32),
            torch.tensor(kvi, dtype=torch.int32), torch.tensor(lpl, dtype=torch.int32), hq, hkv, d, page,
            causal=True, q_data_type=dtype)
-    # 16-bit storage at head_dim 128 with 16-token pages streams (on 3 CUs a workgroup may need more
-    # segments than its table holds: the tile kernel then); other shapes take the tile / VALU kernels
+    # 16-bit storage at head_dim 128 with 16-token pages takes "stream" plans (on 3 CUs a workgroup may need
+    # more segments than its table holds: "tile" then), whose prompts run as blocks or on the streaming kernel
     if dtype == torch.float32:
         assert w.stats.kernel == "valu"
     elif d == 128 and page % 16 == 0:
         assert w.stats.kernel == "stream" or (cus is not None and w.stats.kernel == "tile")
     else:
         assert w.stats.kernel == "tile"
+    out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
+    torch.cuda.synchronize()
+    ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, causal=True)
+    _check(out, lse, ref_o, ref_lse, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", ["fresh_1000", "ragged_batch", "continue_cached"])
+@pytest.mark.parametrize("cus", [None, 3])
+@pytest.mark.parametrize("no_blocks", [False, True])
+def test_long_causal_plans_on_both_kernels(ws, dtype, case, cus, no_blocks):
+    """The plans that may run as blocks, on each of the two kernels: partial
+    slots and the merge on all CUs, long runs on three.  (A three-CU streaming
+    workgroup's table does not hold the ragged batch: blocks again.)"""
+    from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
+    q_lens, kv_lens, hq, hkv, d, page = CASES[case]
+    print(f"[case] prefill {case} {dtype} cus={cus} no_blocks={no_blocks}", flush=True)
+    (qo, kvp, kvi, lpl), pages = _levels(q_lens, kv_lens, page)
+    g = torch.Generator().manual_seed(7)
+    s = 1 / math.sqrt(d)
+    kv = (torch.randn((pages, 2, page, hkv, d), generator=g) * s).to(dtype)
+    q = (torch.randn((qo[-1], hq, d), generator=g) * s).to(dtype)
+    w = BatchPrefillWithPagedKVCacheWrapper(ws)
+    w._num_cus, w._no_blocks = cus, no_blocks
+    w.plan(qo, kvp, kvi, lpl, hq, hkv, d, page, causal=True, q_data_type=dtype)
+    # (200 and 64 tokens after 500 and 33 cached ones stream by default on all CUs)
+    if no_blocks and not (cus and case == "ragged_batch") or not (cus or no_blocks) and case == "continue_cached":
+        assert w.stats.launches == ("attn_stream_kernel", "tail_merge_kernel") and w.stats.num_merge > 0
+    else:
+        assert w.stats.launches == ("attn_block_kernel",)
     out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
     torch.cuda.synchronize()
     ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, causal=True)
