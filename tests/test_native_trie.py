@@ -202,6 +202,40 @@ def test_trie_plan_equals_attn_plan_of_its_metadata(caps):
     assert np.array_equal(plan_a[: info_a.plan_ints], plan_b[: info_b.plan_ints])
 
 
+def test_plan_kind_takes_less_scratch_when_the_plan_does_not_fit():
+    """plan_kind replans with BE_PLAN_LESS_SCRATCH like the wrapper's plan:
+    120 fp32 beams on one prompt, cut into more keys as 64-row items than as
+    32-row ones, in a workspace that only the latter fit."""
+    import types
+
+    from beam_engine_amd.attention import _PagedPlanner
+    pt = make_pt(4096, 16)
+    st = NativeBeamState(120, pt)
+    st.add_root_sequence(list(range(2000)), request_id=0)
+    st.add_filtered_results([BeamGenerateResult(c, [BeamToken(j, -0.1 * j) for j in range(120)]) for c in st.candidates])
+
+    class Wrapper:
+        _caps, _num_cus = None, 256
+        _need, _less_scratch = staticmethod(_PagedPlanner._need), _PagedPlanner._less_scratch
+
+        def __init__(self, nbytes):
+            self._ws = types.SimpleNamespace(numel=lambda: nbytes, device=None)
+
+        def _plan_flags(self):
+            return 0
+
+        def _install_plan(self, info, *a, **k):
+            self.need = self._need(info)
+
+    def need(nbytes):
+        w = Wrapper(nbytes)
+        st.plan_kind(w, "cascade", 32, 8, 128, torch.float32, host_plan=torch.zeros(1 << 18, dtype=torch.int32))
+        return w.need
+    full = need(1 << 40)
+    less = need(full - 1)
+    assert less < full and need(less) == less
+
+
 def _py_levels(st, kind, include_self, picker):
     """The Python restatement's levels of one strategy (BeamState.segment_tree /
     absorb_edges / tree_levels, StrategyPicker.choose)."""
