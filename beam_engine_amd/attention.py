@@ -408,8 +408,9 @@ class BatchPrefillWithPagedKVCacheWrapper(_PagedPlanner):
     r's queries ``q[qo_indptr[r]:qo_indptr[r+1]]`` attend to its pages, whose
     K/V the caller wrote first; ``causal=True`` gives query i of n the first
     kv_len - n + i + 1 tokens.  bf16 / fp16 prompts run as 128-row MFMA blocks
-    (short ones of head_dim 128 on the streaming kernel), fp32 ones on the
-    fp32 MFMA kernel, with a per-row causal limit; query tiles stop at the
+    (at head_dim 128 on the streaming kernel where that is modelled faster: short
+    ones, few new tokens after cached ones), up to 64 query rows a group on the
+    tile kernel, fp32 ones on the fp32 MFMA kernel, with a per-row causal limit; query tiles stop at the
     chunk holding their last visible token."""
 
     def __init__(self, float_workspace_buffer: torch.Tensor, kv_layout: str = "NHD"):

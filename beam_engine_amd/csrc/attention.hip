@@ -1,4 +1,6 @@
-// Paged decode attention for flat / cascade / tree work lists on gfx950.
+// Paged attention over work lists on gfx950: the planner (which also decides for
+// the streaming and row-block kernels), the VALU kernel, the merge kernel and the
+// launches; the MFMA kernels are in attn_tile.hip, attn_block.hip, attn_f32.hip.
 //
 // One work-list format serves every strategy.  A work item is a tile of
 // queries (a contiguous slice of q_index) attending to a contiguous token range

@@ -1,6 +1,7 @@
 // Work-list plans of the per-(item, KV head) attention kernels (gfx950): the
-// plan's records, the kernels' arguments, and the epilogue pieces shared by
-// attention.hip (tile and VALU kernels) and attn_block.hip (128-row blocks).
+// plan's records, the kernels' arguments, the tile loads of attn_tile.hip (up to
+// 64 rows), attn_block.hip (128-row blocks) and attn_f32.hip, and the epilogue
+// pieces they share with attention.hip (the VALU kernel).
 #pragma once
 
 #include "attention.h"
@@ -32,7 +33,7 @@ static_assert(sizeof(WorkItem) == 32, "WorkItem is 8 int32 words");
 constexpr int kTile = 64;              // tokens per LDS tile
 constexpr int kMaxPagesLds = 1024;     // page ids of one item staged in LDS
 constexpr int kMaxRows = 32;       // rows (queries x GQA group) per VALU workgroup
-constexpr int kMaxTileRows = 128;  // rows per MFMA workgroup (8 row tiles of 16)
+constexpr int kMaxTileRows = 128;  // rows per 16-bit MFMA item (above 64: the block kernel)
 
 struct AttnArgs {
   const void* q;

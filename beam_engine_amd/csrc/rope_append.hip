@@ -46,7 +46,8 @@ __device__ __forceinline__ void store4(T* p, const T (&v)[4]) {
 // scalar loads that leave with the row's, and the table entries are the only
 // second trip; a flat thread index took three 64-bit divisions first and looked
 // the page up after the rotation.  MI355X, 128 candidates, 32 / 8 heads, head_dim
-// 128: 4.9 -> 4.6 us per launch.
+// 128: 4.9 -> 4.6 us per launch (a step's eager calls are bound by their host
+// time, about 12 us each, and do not show it).
 template <typename T>
 __global__ __launch_bounds__(256) void rope_append_kernel(const T* qkv, int64_t qkv_sn, int n, int hq, int hkv,
                                                          int d, const int64_t* positions, const T* cos_t,
