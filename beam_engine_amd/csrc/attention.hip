@@ -404,7 +404,7 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   // 9.4 in 4 chunks; after 1000 11.8 and 9.2).
   int64_t causal_chunk = 0, causal_blocks = 0, tiles = 0, queries = 0, span = 0;
   double block_us = 0;
-  if (any_causal && mfma && !less && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
+  if (any_causal && mfma && !less && !caps && rows_cap == kMaxTileRows && block_eligible(dtype, d)) {
     int64_t longest = 0;
     int most_rows = 0;
     std::vector<int64_t> tiles_of;                     // of each query tile

@@ -672,6 +672,20 @@ def test_causal_tile_plans_fill_the_chip(reqs, n, cached, hq, hkv, d, page, item
     assert it[:, 4].sum() == reqs * (n + cached) and (it[:, 3] % 64 == 0).all()
 
 
+def test_fixed_causal_layout_keeps_its_chunks():
+    """Fixed layouts of 16-bit causal plans cut their keys by the general rule,
+    which their capacities were sized for: 9 queries after 1497 cached tokens, 8 / 2
+    heads, head_dim 64, are 8 chunks (12 without the layout)."""
+    _lib, _ = lib()
+    levels = [([0, 9], [0, 48], list(range(48)), [2])]
+    caps = _lib.BePlanCaps(8, 9, 48, 9, 72, 0, 128, 0)
+    rc, info, _, _, L = plan(levels, d=64, page=32, num_pages=48, flags=128, caps=caps)
+    assert rc == 0, L.be_last_error()
+    assert info.num_items == 8
+    rc, info, *_ = plan(levels, d=64, page=32, num_pages=48, flags=128)
+    assert rc == 0 and info.num_items == 12
+
+
 @pytest.mark.parametrize("dtype,d,page,n,cached,flags,launches,chunk", [
     (2, 128, 16, 1000, 0, 128, ("attn_block_kernel",), 1024), (2, 128, 16, 256, 8000, 128, ("attn_block_kernel", "merge_kernel"), None),
     (2, 128, 16, 1000, 0, 128 | 4096, ("attn_stream_kernel", "tail_merge_kernel"), None),
