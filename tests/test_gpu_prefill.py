@@ -89,6 +89,9 @@ def test_prefill_wrapper_causal(ws, dtype, case, cus):
         assert w.stats.kernel == "valu"
     elif d == 128 and page % 16 == 0:
         assert w.stats.kernel == "stream" or (cus is not None and w.stats.kernel == "tile")
+        # (200 and 64 tokens after 500 and 33 cached ones stream on all CUs)
+        streams = case == "continue_cached" and cus is None
+        assert w.stats.launches[0] == ("attn_stream_kernel" if streams else "attn_block_kernel")
     else:
         assert w.stats.kernel == "tile"
     out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
@@ -97,30 +100,28 @@ def test_prefill_wrapper_causal(ws, dtype, case, cus):
     _check(out, lse, ref_o, ref_lse, dtype)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("case", ["fresh_1000", "ragged_batch", "continue_cached"])
-@pytest.mark.parametrize("cus", [None, 3])
-@pytest.mark.parametrize("no_blocks", [False, True])
-def test_long_causal_plans_on_both_kernels(ws, dtype, case, cus, no_blocks):
-    """The plans that may run as blocks, on each of the two kernels: partial
+@pytest.mark.parametrize("case,dtype,cus", [
+    ("fresh_1000", torch.bfloat16, None), ("fresh_1000", torch.bfloat16, 3), ("ragged_batch", torch.float16, None),
+    ("ragged_batch", torch.float16, 3), ("continue_cached", torch.bfloat16, 3)])
+def test_long_causal_plans_without_blocks(ws, case, dtype, cus):
+    """Plans that run as blocks by default, on the streaming kernel: partial
     slots and the merge on all CUs, long runs on three.  (A three-CU streaming
     workgroup's table does not hold the ragged batch: blocks again.)"""
     from beam_engine_amd import BatchPrefillWithPagedKVCacheWrapper
     q_lens, kv_lens, hq, hkv, d, page = CASES[case]
-    print(f"[case] prefill {case} {dtype} cus={cus} no_blocks={no_blocks}", flush=True)
+    print(f"[case] prefill {case} {dtype} cus={cus} without blocks", flush=True)
     (qo, kvp, kvi, lpl), pages = _levels(q_lens, kv_lens, page)
     g = torch.Generator().manual_seed(7)
     s = 1 / math.sqrt(d)
     kv = (torch.randn((pages, 2, page, hkv, d), generator=g) * s).to(dtype)
     q = (torch.randn((qo[-1], hq, d), generator=g) * s).to(dtype)
     w = BatchPrefillWithPagedKVCacheWrapper(ws)
-    w._num_cus, w._no_blocks = cus, no_blocks
+    w._num_cus, w._no_blocks = cus, True
     w.plan(qo, kvp, kvi, lpl, hq, hkv, d, page, causal=True, q_data_type=dtype)
-    # (200 and 64 tokens after 500 and 33 cached ones stream by default on all CUs)
-    if no_blocks and not (cus and case == "ragged_batch") or not (cus or no_blocks) and case == "continue_cached":
-        assert w.stats.launches == ("attn_stream_kernel", "tail_merge_kernel") and w.stats.num_merge > 0
-    else:
+    if cus and case == "ragged_batch":
         assert w.stats.launches == ("attn_block_kernel",)
+    else:
+        assert w.stats.launches == ("attn_stream_kernel", "tail_merge_kernel") and w.stats.num_merge > 0
     out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
     torch.cuda.synchronize()
     ref_o, ref_lse = oa.cascade_attention(q, kv, [qo], [kvp], [kvi], [lpl], page, causal=True)
