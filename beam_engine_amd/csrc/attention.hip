@@ -538,14 +538,12 @@ int attn_plan(const be_level* levels, int num_levels, int num_queries, int hq, i
   if (any_causal)
     std::stable_sort(items.begin(), items.end(), [](const WorkItem& x, const WorkItem& y) { return x.tok_count > y.tok_count; });
 
-  // ---- merge list (queries with >= 2 partial rows) and zero list (no keys)
+  // ---- merge list (queries with partial rows: one of a tile whose other queries
+  // have more items has a row too, if only one) and zero list (no keys)
   std::vector<int> merge_q, merge_ptr{0}, merge_rows, zero_q;
   for (int qi = 0; qi < num_queries; ++qi) {
-    if (cnt[qi] == 1) continue;
-    if (cnt[qi] == 0) {
-      zero_q.push_back(qi);
-      continue;
-    }
+    if (cnt[qi] == 0) zero_q.push_back(qi);
+    if (rows_of[qi].empty()) continue;
     merge_q.push_back(qi);
     for (int r : rows_of[qi]) merge_rows.push_back(r);
     merge_ptr.push_back((int)merge_rows.size());

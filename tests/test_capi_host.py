@@ -4,6 +4,7 @@ planner (host code) validates its inputs and produces a consistent work list."""
 
 import ctypes
 import os
+import random
 import re
 
 import numpy as np
@@ -670,6 +671,52 @@ def test_causal_tile_plans_fill_the_chip(reqs, n, cached, hq, hkv, d, page, item
     assert info.kernel == 1 and info.tile_rows <= 64 and info.num_items == items
     it = decode_items(info, buf)
     assert it[:, 4].sum() == reqs * (n + cached) and (it[:, 3] % 64 == 0).all()
+
+
+@pytest.mark.parametrize("seed", range(120))
+def test_every_query_is_written_once(seed):
+    """Work-list plans of random levels (groups of different sizes, empty ones,
+    causal or not): a query's partial rows are merged however many they are, a
+    query without rows is written by exactly one direct item, one without any
+    item is on the zero list."""
+    r = random.Random(seed)
+    dtype, d, page = r.choice([(0, 128, 16), (1, 128, 8), (2, 64, 16), (2, 256, 16), (1, 64, 3), (2, 128, 16)])
+    hkv = r.choice([1, 2, 8])
+    hq, nq, nlv, pages = hkv * r.choice([1, 4, 5]), r.randint(1, 200), r.randint(1, 3), 0
+    levels = []
+    for _ in range(nlv):
+        qo, kvp, kvi, lpl = [0], [0], [], []
+        while qo[-1] < nq:
+            n = min(nq - qo[-1], r.choice([1, 1, 2, 5, 17, 64, 200]))
+            kv = r.choice([0, 1, r.randint(1, 40), r.randint(1, 4000), n, max(1, n // 2)])
+            npg = -(-kv // page)
+            kvi += list(range(pages, pages + npg))
+            pages += npg
+            qo.append(qo[-1] + n)
+            kvp.append(len(kvi))
+            lpl.append(kv - (npg - 1) * page if npg else 0)
+        levels.append((qo, kvp, kvi, lpl))
+    flags = (128 if r.random() < 0.6 else 0) | TILE | (2 if r.random() < 0.3 else 0) | (8192 if r.random() < 0.3 else 0)
+    rc, info, buf, _lib, L = plan(levels, nq=nq, hq=hq, hkv=hkv, d=d, page=page, num_pages=max(pages, 1), dtype=dtype, flags=flags,
+                                  cus=r.choice([3, 16, 256]))
+    assert rc == 0, L.be_last_error()
+    direct, rows = np.zeros(nq, int), {}
+    for q0, qn, _, _, _, orow, _, _ in decode_items(info, buf).tolist():
+        for j in range(qn):
+            if orow < 0:
+                direct[q0 + j] += 1
+            else:
+                rows.setdefault(q0 + j, []).append(orow + j)
+    mq = buf[info.off_merge_q: info.off_merge_q + info.num_merge].tolist()
+    mp = buf[info.off_merge_ptr: info.off_merge_ptr + info.num_merge + 1]
+    mr = buf[info.off_merge_rows:]
+    assert mq == sorted(rows)
+    for i, q in enumerate(mq):
+        assert sorted(mr[mp[i]: mp[i + 1]].tolist()) == sorted(rows[q]) and direct[q] == 0
+        assert buf[info.off_q_merge + q] == i
+    zero = set(buf[info.off_zero_q: info.off_zero_q + info.num_zero].tolist())
+    for q in range(nq):
+        assert (q in rows) + (direct[q] == 1) + (q in zero) == 1 and direct[q] <= 1
 
 
 def test_fixed_causal_layout_keeps_its_chunks():

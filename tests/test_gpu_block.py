@@ -237,6 +237,31 @@ def test_fp32_fixed_layout(ws, tile_rows):
     _check(out, lse, ref_o, ref_lse, torch.float32)
 
 
+@pytest.mark.parametrize("dtype,d,page", [(torch.bfloat16, 128, 8), (torch.float32, 128, 16), (torch.float16, 64, 16),
+                                          (torch.bfloat16, 256, 16)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_queries_with_one_item_beside_others(ws, dtype, d, page, fused):
+    """Two levels on the work-list kernels, some queries without keys on the
+    second or the first: a query's only item may share its tile with queries of
+    more items, and its partial row is the whole result."""
+    from beam_engine_amd import MultiLevelCascadeAttentionWrapper
+    print(f"[case] one item beside others {dtype} d {d} page {page} fused {fused}", flush=True)
+    hq, hkv, nq = 8, 2, 24
+    (qo0, kvp0, kvi0, lpl0), p0 = _levels([16, 8], [700, 0], page)
+    (qo1, kvp1, kvi1, lpl1), p1 = _levels([1] * nq, [0 if i % 3 == 0 else 5 + 11 * i for i in range(nq)], page)
+    levels = ([qo0, qo1], [kvp0, kvp1], [kvi0, [p0 + x for x in kvi1]], [lpl0, lpl1])
+    g = torch.Generator().manual_seed(12)
+    kv = torch.randn((p0 + p1, 2, page, hkv, d), generator=g).to(dtype)
+    q = torch.randn((nq, hq, d), generator=g).to(dtype)
+    w = MultiLevelCascadeAttentionWrapper(2, ws)
+    w._fused_merge = fused
+    w.plan(*levels, hq, hkv, d, page, q_data_type=dtype)
+    out, lse = w.run(q.cuda(), kv.cuda(), return_lse=True)
+    torch.cuda.synchronize()
+    ref_o, ref_lse = oa.cascade_attention(q, kv, *levels, page)
+    _check(out, lse, ref_o, ref_lse, dtype)
+
+
 @pytest.mark.parametrize("dtype,d,page,n,hq", [
     (torch.float32, 64, 16, 2, 8), (torch.float32, 128, 3, 8, 8), (torch.float32, 256, 8, 30, 8), (torch.bfloat16, 64, 8, 2, 8),
     (torch.bfloat16, 256, 3, 20, 8), (torch.float16, 128, 8, 8, 8), (torch.float16, 64, 16, 40, 8), (torch.bfloat16, 128, 5, 90, 8)])
