@@ -1664,9 +1664,12 @@ __device__ __forceinline__ void row_sum(bool in, float mu, double su, bool again
   B = __shfl(wave_scan_add_f64(t), 63, 64);
 }
 
-// L = fl32(ln S) from row_sum's values.
+// L = fl32(ln S) from row_sum's values.  S is taken before its logarithm: log(B) +
+// (R - mm) would round at the magnitude of mm, which a row whose best logit holds
+// nearly all the mass shows (logits up to 400: its log-probability 0 instead of
+// -1.8e-15).
 __device__ __forceinline__ float row_log(float mm, float R, double B) {
-  return (float)(log(B) + ((double)R - (double)mm));
+  return (float)log(B * exp((double)R - (double)mm));
 }
 
 // Pass 3 for request q (rows [rb, re)) from the row lists written by this

@@ -344,3 +344,30 @@ def test_segment_with_more_candidates_than_its_space(dtype):
     x[2, lane % 64 == 3] += 30.0
     x[3, :3000] += 50.0
     compare(x.to(dtype), [0.0, -0.5, -1.0, -1.5], 8)
+
+
+@pytest.mark.parametrize("n,v,beam,kind", [(16, 1735, 16, "spread"), (32, 467, 32, "spread"), (6, 34943, 3, "spread"),
+                                           (32, 47896, 32, "spread"), (4, 128256, 4, "peak"), (2, 8000, 8, "peak")])
+def test_rows_that_one_logit_dominates(n, v, beam, kind):
+    """Rows whose best logit holds nearly all the mass (16-bit logits up to some
+    400, or 40 ahead of the rest): their log-probabilities near zero come from the
+    sum of exponentials, not from its logarithm less the maximum.  2^-47: 64
+    half-ulp roundings of a sum near 1 (a thread adds 32, the waves, segments and
+    the scale some twenty)."""
+    from beam_engine_amd import beam_topk, decode_k
+    say(f"topk dominated rows {n} x {v} beam {beam} {kind}")
+    g = torch.Generator().manual_seed(n + v)
+    x = torch.randn((n, v), generator=g) * (120.0 if kind == "spread" else 2.0)
+    if kind == "peak":
+        x[torch.arange(n), torch.arange(n) * 7] += 40.0
+    x = x.to(torch.bfloat16)
+    k = decode_k(beam, v)
+    vals, idx = ot.row_topk(ot.log_softmax_rows(x.float().numpy(), "bfloat16", 1.0), k)
+    rv, ri = beam_topk(x.cuda(), k)
+    torch.cuda.synchronize()
+    assert np.array_equal(ri.cpu().numpy(), idx)
+    rv = rv.cpu().numpy()
+    small = np.abs(vals) < 1e-6
+    assert small.any()
+    assert np.abs(rv[small].astype(np.float64) - vals[small]).max() <= 2.0 ** -47
+    assert np.array_equal(rv[~small].view(np.uint32), vals[~small].view(np.uint32))
