@@ -1667,9 +1667,11 @@ __device__ __forceinline__ void row_sum(bool in, float mu, double su, bool again
 // L = fl32(ln S) from row_sum's values.  S is taken before its logarithm: log(B) +
 // (R - mm) would round at the magnitude of mm, which a row whose best logit holds
 // nearly all the mass shows (logits up to 400: its log-probability 0 instead of
-// -1.8e-15).
+// -1.8e-15).  Within the two products' rounding of 1 it is 1: a row that holds
+// one logit's mass only has L = 0, and no log-probability is above 0.
 __device__ __forceinline__ float row_log(float mm, float R, double B) {
-  return (float)log(B * exp((double)R - (double)mm));
+  const double s = B * exp((double)R - (double)mm);
+  return fabs(s - 1.0) <= 0x1.8p-52 ? 0.0f : (float)log(s);
 }
 
 // Pass 3 for request q (rows [rb, re)) from the row lists written by this
