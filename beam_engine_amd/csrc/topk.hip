@@ -1080,12 +1080,17 @@ __global__ __launch_bounds__(kTopkThreads) void topk_row_kernel(const T* logits,
 }
 
 // ---------------------------------------------------------------- pass 3
+// What a pool total is ordered by.
+__device__ __forceinline__ double pool_key(double t) { return t == t ? t : -INFINITY; }
+
 // Per request: the beam best of its pool total = parent[r] + (double)row_vals[r, j]
 // by (total desc, pool position r * k + j asc), emitted grouped by row.  Each
 // row's list is sorted by logp desc (its totals do not increase along it), so
 // an entry's pool rank is its rank in its row plus, in every other row, the
 // entries that precede it (a binary search); entries j >= beam of a row
-// cannot be selected.
+// cannot be selected.  A NaN total (a row of -inf logits, a NaN parent score)
+// ranks as -inf and is emitted as it is: compared as a NaN it would precede
+// nothing and follow nothing, and every such entry would be among the best.
 __global__ __launch_bounds__(kTopkThreads) void topk_pool_kernel(int n_rows, int k, int beam, const int32_t* req_row_ptr,
                                                                 const double* parent, const float* row_vals,
                                                                 const int32_t* row_idx, int32_t* out_parent,
@@ -1115,7 +1120,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_pool_kernel(int n_rows, int
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int i = i0 + u * kTopkThreads + tid;
-      if (i < n) tot[i] = pv[u] + (double)rv[u];
+      if (i < n) tot[i] = pool_key(pv[u] + (double)rv[u]);
     }
   }
   for (int i = tid; i < nr; i += kTopkThreads) sel[i] = 0;
@@ -1168,9 +1173,11 @@ __global__ __launch_bounds__(kTopkThreads) void topk_pool_kernel(int n_rows, int
     const int rr = e / jb, j = e - rr * jb;
     if (j < sel[rr]) {
       const int at = first[rr] + j;
+      if (at >= beam) continue;                        // (a list that is not in order: NaN among its values)
+      const double t = tot[rr * k + j];
       op[at] = rb + rr;
       ot[at] = row_idx[(int64_t)(rb + rr) * k + j];
-      os[at] = tot[rr * k + j];
+      os[at] = t != -INFINITY ? t : parent[rb + rr] + (double)row_vals[(int64_t)(rb + rr) * k + j];
     }
   }
   for (int i = first[nr] + tid; i < beam; i += kTopkThreads) {
@@ -1679,18 +1686,21 @@ __device__ __forceinline__ float row_log(float mm, float R, double B) {
 // thread of the block; ends with a barrier).  An entry's rank is its position
 // in its row plus, in every other row, the entries before it in the order
 // (total desc, pool position asc) -- a prefix of that row, found by binary
-// search; P adjacent threads share an entry, each taking every P-th row.
+// search; P adjacent threads share an entry, each taking every P-th row.  NaN
+// totals as in topk_pool_kernel.
 __device__ void fused_pool(const FusedTopkArgs& a, int rb, int re, int q, RowLds& sm) {
   const int tid = threadIdx.x, k = a.k, beam = a.beam;
   int32_t* op = a.out_parent + (int64_t)q * beam;
   int32_t* ot = a.out_token + (int64_t)q * beam;
   double* os = a.out_score + (int64_t)q * beam;
   const int nr = re - rb, jb = min(k, beam), n = nr * jb;
+  double score = 0.0;                                  // entry tid's total
   if (tid < n) {
     const int rr = tid / jb, j = tid - rr * jb;
     const float rv = ld_co(a.row_vals + (int64_t)(rb + rr) * k + j);
     const int32_t ri = ld_co(a.row_idx + (int64_t)(rb + rr) * k + j);
-    sm.ptot[tid] = a.parent[rb + rr] + (double)rv;
+    score = a.parent[rb + rr] + (double)rv;
+    sm.ptot[tid] = pool_key(score);
     sm.pidx[tid] = ri;
   }
   for (int i = tid; i < nr; i += kRowThreads) sm.sel[i] = 0;
@@ -1834,11 +1844,11 @@ __device__ void fused_pool(const FusedTopkArgs& a, int rb, int re, int q, RowLds
   __syncthreads();
   if (tid < n) {
     const int r2 = tid / jb, j2 = tid - r2 * jb;
-    if (j2 < sm.sel[r2]) {
-      const int at = sm.first[r2] + j2;
+    const int at = sm.first[r2] + j2;
+    if (j2 < sm.sel[r2] && at < beam) {
       op[at] = rb + r2;
       ot[at] = sm.pidx[tid];
-      os[at] = sm.ptot[tid];
+      os[at] = score;
     }
   }
   for (int i = sm.first[nr] + tid; i < beam; i += kRowThreads) {

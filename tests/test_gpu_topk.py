@@ -371,3 +371,55 @@ def test_rows_that_one_logit_dominates(n, v, beam, kind):
     assert small.any()
     assert np.abs(rv[small].astype(np.float64) - vals[small]).max() <= 2.0 ** -47
     assert np.array_equal(rv[~small].view(np.uint32), vals[~small].view(np.uint32))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,v,beam", [((32,), 42, 32), ((48, 2), 300, 16), ((3, 128, 1), 600, 16), ((2, 5), 9, 4),
+                                         ((16, 16), 40000, 16)])
+@pytest.mark.parametrize("dead", ["all", "odd", "parent"])
+def test_rows_without_a_probability(dtype, rows, v, beam, dead):
+    """Rows of -inf logits (log-probabilities NaN: a mask that leaves no token)
+    and rows under a NaN parent score: their totals rank as -inf, every request
+    writes its beam entries and nothing past them (two and three kernels; 32
+    rows x 32 fill the pool), and the other rows are chosen as without them."""
+    from beam_engine_amd import _lib, decode_k
+    say(f"topk dead rows {rows} x {v} beam {beam} {dtype} {dead}")
+    n, k = sum(rows), decode_k(beam, v)
+    g = torch.Generator().manual_seed(n + v)
+    logits = (torch.randn((n, v), generator=g) * 2).to(dtype)
+    parents = -torch.rand(n, generator=g, dtype=torch.float64) * 3
+    bad = torch.arange(n) % 2 == 1 if dead != "all" else torch.ones(n, dtype=torch.bool)
+    if dead == "parent":
+        parents[bad] = float("nan")
+    else:
+        logits[bad] = float("-inf")
+    lib = _lib.load()
+    dl, dp = logits.cuda(), parents.cuda()
+    ptr = torch.tensor(np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)).cuda()
+    ws = torch.empty(lib.be_beam_topk_workspace_bytes(n, v, k), dtype=torch.uint8, device="cuda")
+    rv = torch.empty((n, k), dtype=torch.float32, device="cuda")
+    ri = torch.empty((n, k), dtype=torch.int32, device="cuda")
+    m, guard = len(rows) * beam, n * k                 # room for every entry of the pool after the outputs
+    par = torch.full((m + guard,), -77, dtype=torch.int32, device="cuda")
+    tok = torch.full((m + guard,), -77, dtype=torch.int32, device="cuda")
+    sc = torch.full((m + guard,), -77.0, dtype=torch.float64, device="cuda")
+    _lib.check(lib.be_beam_topk(dl.data_ptr(), _lib.dtype_code(dtype), n, v, v, 1.0, 0, k, dp.data_ptr(), beam,
+                                len(rows), ptr.data_ptr(), max(rows), rv.data_ptr(), ri.data_ptr(), par.data_ptr(),
+                                tok.data_ptr(), sc.data_ptr(), ws.data_ptr(), ws.numel(),
+                                _lib.stream_ptr(dl.device)), "beam top-k")
+    torch.cuda.synchronize()
+    assert (par[m:] == -77).all() and (tok[m:] == -77).all() and (sc[m:] == -77.0).all()
+    with np.errstate(invalid="ignore", divide="ignore"):
+        vals, idx = ot.row_topk(ot.log_softmax_rows(logits.float().numpy(), DT[dtype]), k)
+    assert np.array_equal(ri.cpu().numpy(), idx)
+    assert np.array_equal(rv.cpu().numpy(), vals, equal_nan=True)
+    b = 0
+    for q, r in enumerate(rows):
+        pool = [(i, int(idx[i, j]), float(parents[i]) + float(vals[i, j])) for i in range(b, b + r) for j in range(k)]
+        best = sorted(pool, key=lambda e: -e[2] if e[2] == e[2] else float("inf"))[:beam]       # (stable)
+        best.sort(key=lambda e: e[0])
+        at = slice(q * beam, q * beam + len(best))
+        assert par[at].tolist() == [e[0] for e in best] and tok[at].tolist() == [e[1] for e in best], q
+        assert np.array_equal(sc[at].cpu().numpy(), np.array([e[2] for e in best]), equal_nan=True), q
+        assert (par[at.stop:(q + 1) * beam] == -1).all()
+        b += r
