@@ -1039,7 +1039,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_row_kernel(const T* logits,
       if (bk != 0 && key_of_x(bk) >= kth) atomicOr(&flag, 1);
     }
     __syncthreads();
-    exact = flag != 0 || ntie > kMaxTie;
+    // (fewer than k with the ties: NaN logps, whose order is not that of x')
+    exact = flag != 0 || ntie > kMaxTie || nfin + ntie < k;
     if (!exact) {
       const int above = nfin, g = ntie, need = k - above;
       for (int i = tid; i < g; i += kTopkThreads) {
@@ -1966,12 +1967,16 @@ __global__ __launch_bounds__(kRowThreads) void topk_rows16_kernel(FusedTopkArgs 
   if (!exact0) {
     // the k-th largest x' key: radix passes over the keys' offsets from lo
     // (one pass when the range spans at most 256 keys), while wave 0 takes
-    // the row's log-sum-exp
+    // the row's log-sum-exp.  (A key past the last bin is a NaN logit's: the
+    // row max leaves NaN out.  Without it the bins may hold fewer than k, and
+    // the counts below tell whether the k-th they give is the k-th.)
     const uint32_t lo = (uint32_t)sm.lo;
     const int shift = sm.shift;
 #pragma unroll
-    for (int q = 0; q < PER; ++q)
-      if (xk[q] >= lo && xk[q] != 0) atomicAdd(&sm.hist[0][(xk[q] - lo) >> shift], 1);
+    for (int q = 0; q < PER; ++q) {
+      const uint32_t bin = (xk[q] - lo) >> shift;
+      if (xk[q] >= lo && xk[q] != 0 && bin < 256u) atomicAdd(&sm.hist[0][bin], 1);
+    }
     __syncthreads();
     if (w == 0 && lane == 0) {
       sm.m = mm_row;
@@ -2018,7 +2023,8 @@ __global__ __launch_bounds__(kRowThreads) void topk_rows16_kernel(FusedTopkArgs 
       const uint32_t lk = logp_key16<T>(value_of_key16<T>(xk[q]), m, L);
       const uint64_t e = ((uint64_t)lk << 32) | (uint32_t)cv[q];
       if (lk > K) {
-        sm.fin[atomicAdd(&sm.nabove, 1)] = e;
+        const int at = atomicAdd(&sm.nabove, 1);
+        if (at < k) sm.fin[at] = e;
       } else if (lk == K) {
         const int at = atomicAdd(&sm.ntie, 1);
         if (at < kFusedTie) sm.tg[at] = e;
@@ -2029,7 +2035,9 @@ __global__ __launch_bounds__(kRowThreads) void topk_rows16_kernel(FusedTopkArgs 
       if (bd != 0 && logp_key16<T>(value_of_key16<T>(bd), m, L) >= K) atomicOr(&sm.exact, 1);
     }
     __syncthreads();
-    if (!sm.exact && sm.ntie <= kFusedTie) {
+    // (fewer than k above K and k with its ties: anything else means NaN logps,
+    // whose order is not that of x')
+    if (!sm.exact && sm.ntie <= kFusedTie && sm.nabove < k && sm.nabove + sm.ntie >= k) {
       // the need lowest indices of the tie group (largest composite keys)
       const int above = sm.nabove, g = sm.ntie, need = k - above;
       if (g <= 32) {

@@ -423,3 +423,38 @@ def test_rows_without_a_probability(dtype, rows, v, beam, dead):
         assert np.array_equal(sc[at].cpu().numpy(), np.array([e[2] for e in best]), equal_nan=True), q
         assert (par[at.stop:(q + 1) * beam] == -1).all()
         b += r
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("v,beam", [(700, 4), (5000, 16), (128256, 32)])
+def test_nan_and_infinite_logits(dtype, v, beam):
+    """Rows with a NaN (the row max leaves it out, so its key lies past every
+    bin of the row's key range), with more NaN of a lower payload than the list
+    holds, with +inf, and wholly NaN (both signs, the pattern that marks
+    positions past a segment among them): a list of k different tokens, and a
+    row without them beside them is selected as ever."""
+    from beam_engine_amd import beam_topk, decode_k
+    say(f"topk nan logits 7 x {v} beam {beam} {dtype}")
+    k = decode_k(beam, v)
+    g = torch.Generator().manual_seed(v)
+    logits = (torch.randn((7, v), generator=g) * 2).to(dtype)
+    it = torch.int32 if dtype == torch.float32 else torch.int16
+    bits = logits.view(it)
+    quiet = {torch.bfloat16: 0x7fc0, torch.float16: 0x7e00, torch.float32: 0x7fc00000}[dtype]
+    bits[0, v // 3] = quiet
+    bits[1, 5:5 + k // 2] = quiet + 3
+    bits[1, v // 2:v // 2 + 300] = quiet + 1
+    logits[2, v - 2] = float("inf")
+    bits[3, :] = quiet
+    bits[4, :] = -1
+    bits[5, ::3] = -1
+    parents = torch.zeros(7, dtype=torch.float64)
+    rv, ri, (par, tok, sc) = beam_topk(logits.cuda(), k, parents, beam, request_rows=[1] * 7)
+    torch.cuda.synchronize()
+    ri = ri.cpu()
+    for r in range(7):
+        assert ri[r].min() >= 0 and ri[r].max() < v and ri[r].unique().numel() == k, f"row {r}"
+    par, tok = par.reshape(7, beam).cpu(), tok.reshape(7, beam).cpu()
+    assert ((par == torch.arange(7)[:, None]) | (par == -1)).all() and (tok < v).all()
+    _, _, _, _, flat = ot.beam_step(logits[6:].float().numpy(), [0.0], beam, DT[dtype])
+    assert tok[6].tolist() == [e[1] for e in flat] and sc.reshape(7, beam)[6].tolist() == [e[2] for e in flat]
