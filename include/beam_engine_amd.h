@@ -483,7 +483,7 @@ int be_merge_states(const float* o_a, const float* lse_a, const float* o_b, cons
  *   [req_row_ptr[q], req_row_ptr[q+1]), a device int32 array; NULL with
  *   n_req = 1 means all rows): the beam best of the request's pool
  *   total = parent_scores[r] + (double)row_vals[r, j] by (total desc,
- *   r*k + j asc), emitted grouped by row ascending and, within a row, in
+ *   r*k + j asc; a NaN total ranks as -inf), emitted grouped by row ascending and, within a row, in
  *   selection order, into out_parent (global row) / out_token (int32) and
  *   out_score (double) [n_req * beam].  max_req_rows bounds the rows of any
  *   request (host-side pool capacity check).
